@@ -27,6 +27,7 @@
 #include "st_fftlds.h"
 #include "st_track_common.h"
 #include "st_fftreg.h"
+#include "st_fft8.h"
 
 using namespace sttrack;
 
@@ -38,6 +39,9 @@ __constant__ double2 c_root256[256];
 namespace fftreg {
 __constant__ float2 c_tw128[128];
 }  // namespace fftreg
+namespace fft8 {
+__constant__ float2 c_tw256[256];
+}  // namespace fft8
 
 // global-address-space views of pointers held in parameter blocks (loads
 // through them are global loads, not flat ones that also count against
@@ -925,6 +929,9 @@ struct AmpBatch {
     double2 *ppart;  // power partials [B][nPd]
     double2 *mean;   // amplitude means [B]
     Top2 *part;      // coarse top two [B][nPm]
+    // fused path only (the fields above from I to mag, dpart to part unused)
+    float *nb;       // [B][kNbc] |s| around each coarse peak (kNbMap)
+    uint8_t *have;   // [B] 1: matched, for k_cpx_refine
 };
 
 __global__ void __launch_bounds__(NT) k_amp_gather(KPar P, Pts S, const int *list, int off, int B, int large,
@@ -2232,7 +2239,7 @@ __global__ void k_amp_psum(const double2 *ppart, int nPf, int B, int WA, int WR,
 // as scalars, the 8 x 8 boxes (times b) through LDS, and wave 0 merges each
 // attempt's 48 column results and writes them.
 constexpr int kRefPer = 4, kRefThreads = kRefPer * kFine;
-__global__ void __launch_bounds__(kRefThreads) k_cpx_refine(CpxBatch C, int count, int WW)
+__global__ void __launch_bounds__(kRefThreads) k_cpx_refine(CpxBatch C, int count, int WW, int mode)
 {
     __shared__ double2 Pc[kRefPer][NFAST * NFAST];
     __shared__ double s1[kRefThreads], s2[kRefThreads];
@@ -2292,8 +2299,11 @@ __global__ void __launch_bounds__(kRefThreads) k_cpx_refine(CpxBatch C, int coun
     }
     const int iF = I * NOVER + (fi + 24) - (NOVER * NFAST) / 2;
     const int jF = J * NOVER + (fj + 24) - (NOVER * NFAST) / 2;
-    const int cI = iF / NOVER, cJ = jF / NOVER;
-    const bool ok = (cI - NGAUSS / 2) >= 0 && (cI + NGAUSS / 2) < WW && (cJ - NGAUSS / 2) >= 0 &&
+    // mode 0 (complex match): the width samples sit at the refined peak; mode 1
+    // (amplitude try): at the coarse one, with ampTrackFast's edge rule
+    const int cI = mode ? I : iF / NOVER, cJ = mode ? J : jF / NOVER;
+    const int e0 = mode ? 1 : 0;
+    const bool ok = (cI - NGAUSS / 2) >= e0 && (cI + NGAUSS / 2) < WW && (cJ - NGAUSS / 2) >= e0 &&
                     (cJ + NGAUSS / 2) < WW;
     if (l == 0) {
         res->fi = fi;
@@ -2970,6 +2980,8 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
     }
 }
 
+#include "st_amp_fused.h"
+
 // ---------------------------------------------------------------------
 // host side
 
@@ -3105,6 +3117,10 @@ void init_dirichlet(st_ctx *ctx)
     for (int j = 0; j < 128; j++)
         t128[j] = make_float2((float)cos(2.0 * M_PI * j / 128.0), (float)sin(2.0 * M_PI * j / 128.0));
     ST_HIP(hipMemcpyToSymbol(HIP_SYMBOL(fftreg::c_tw128), t128, sizeof(t128)));
+    float2 t256[256];
+    for (int j = 0; j < 256; j++)
+        t256[j] = make_float2((float)cos(-2.0 * M_PI * (double)j / 256.0), (float)sin(-2.0 * M_PI * (double)j / 256.0));
+    ST_HIP(hipMemcpyToSymbol(HIP_SYMBOL(fft8::c_tw256), t256, sizeof(t256)));
     double2 r256[256];
     for (int j = 0; j < 256; j++)
         r256[j] = make_double2(cos(2.0 * M_PI * j / 256.0), sin(2.0 * M_PI * j / 256.0));
@@ -3760,7 +3776,7 @@ struct StrackJob {
             const int kRef = ctx->kernel_slot("k_cpx_refine");
             ctx->time_begin(kRef);
             hipLaunchKernelGGL(k_cpx_refine, dim3((nCpx + kRefPer - 1) / kRefPer), dim3(kRefThreads), 0, st, C,
-                               nCpx, 2 * w);
+                               nCpx, 2 * w, 0);
             ctx->time_end(kRef);
             hipLaunchKernelGGL(k_lm, dim3((2 * nCpx + 127) / 128), dim3(128), 0, st, C.res, nCpx, C.sig);
             hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + 127) / 128), dim3(128), 0, st, P, S, list, 0, nCpx, C);
@@ -3852,11 +3868,66 @@ struct StrackJob {
         const int kRef = ctx->kernel_slot("k_cpx_refine");
         ctx->time_begin(kRef);
         hipLaunchKernelGGL(k_cpx_refine, dim3((nCpx + kRefPer - 1) / kRefPer), dim3(kRefThreads), 0, st, C, nCpx,
-                           2 * w);
+                           2 * w, 0);
         ctx->time_end(kRef);
         hipLaunchKernelGGL(k_lm, dim3((2 * nCpx + 127) / 128), dim3(128), 0, st, C.res, nCpx, C.sig);
         hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + 127) / 128), dim3(128), 0, st, P, S, list, 0, nCpx, C);
         ST_HIP(hipGetLastError());
+    }
+
+    // Whether a try (large: the doubled window) runs on the fused amplitude
+    // kernel: square patches of 16, 32 or 64 samples, whose four planes fit a
+    // CU's LDS; -gauss fits its peak on the staged path's surfaces.
+    bool amp_fused(int large) const
+    {
+        const int ws = pp->wAa * (large ? LA : 1);
+        return pp->wAa == pp->wRa && (ws == 16 || ws == 32 || ws == 64) && !gauss && !staged_only();
+    }
+
+    // Scratch of the fused amplitude path per try.
+    static constexpr size_t kAmpFusedPer =
+        sizeof(PeakRes) + 2 * sizeof(float) + 2 * sizeof(double) + 2 + kNbc * sizeof(float);
+
+    // nA tries of one window on the fused amplitude kernel, refinement, width
+    // fits and acceptance.
+    void amp_alone_fused(int large, int nA)
+    {
+        hipStream_t st = ctx->stream;
+        Arena &ar = ctx->arena;
+        const int sc = large ? LA : 1, ws = pp->wAa * sc;
+        const size_t kMaxBatch = 65536;  // a cancelled job leaves between batches
+        const size_t room = (ar.cap - ar.used - 8 * 256) / kAmpFusedPer;
+        const int B = (int)std::max<size_t>(1, std::min<size_t>({(size_t)nA, room, kMaxBatch}));
+        AmpBatch A{};
+        A.res = ar.take<PeakRes>(B);
+        A.sig = ar.take<float>(2 * (size_t)B);
+        A.p = ar.take<double>(2 * (size_t)B);
+        A.state = ar.take<uint8_t>(B);
+        A.have = ar.take<uint8_t>(B);
+        A.nb = ar.take<float>((size_t)B * kNbc);
+        CpxBatch C{};  // what k_cpx_refine reads
+        C.res = A.res;
+        C.have = A.have;
+        C.nb = A.nb;
+        for (int off = 0; off < nA; off += B) {
+            ctx->check_cancel();
+            const int nb = std::min(B, nA - off);
+            ctx->time_begin(kAmpDet);
+            if (ws == 16)
+                launch_amp_fused<16>(ctx, P, S, list + off, nb, sc, A);
+            else if (ws == 32)
+                launch_amp_fused<32>(ctx, P, S, list + off, nb, sc, A);
+            else
+                launch_amp_fused<64>(ctx, P, S, list + off, nb, sc, A);
+            ctx->time_end(kAmpDet);
+            ctx->time_begin(kAmpPeak);
+            hipLaunchKernelGGL(k_cpx_refine, dim3((nb + kRefPer - 1) / kRefPer), dim3(kRefThreads), 0, st, C, nb, 2 * ws,
+                               1);
+            ctx->time_end(kAmpPeak);
+            hipLaunchKernelGGL(k_lm, dim3((2 * nb + 127) / 128), dim3(128), 0, st, A.res, nb, A.sig);
+            hipLaunchKernelGGL(k_amp_finalize, dim3((nb + 127) / 128), dim3(128), 0, st, P, S, list, off, nb, large, A);
+            ST_HIP(hipGetLastError());
+        }
     }
 
     // Carry of the azimuth shift, amplitude retries, composition, the
@@ -3885,6 +3956,13 @@ struct StrackJob {
             const int nA = read_count(ctx, S.counts, CNT_LIST);
             if (nA == 0)
                 break;
+            if (amp_fused(large)) {
+                amp_alone_fused(large, nA);
+                ar.used = mark;
+                if (!large)
+                    ST_HIP(hipEventRecord(sev[3], st));
+                continue;
+            }
             // patches wsA x wsR, interpolated surfaces WA x WR
             const int wsA = par.wAa * (large ? LA : 1), wsR = par.wRa * (large ? LA : 1), WA = 2 * wsA, WR = 2 * wsR;
             ST_REQUIRE(WA <= kStElems && WR <= kStElems, ST_ERR_UNSUPPORTED,
