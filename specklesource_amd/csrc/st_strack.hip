@@ -2981,6 +2981,7 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
 }
 
 #include "st_amp_fused.h"
+#include "st_amp_large.h"
 
 // ---------------------------------------------------------------------
 // host side
@@ -3976,9 +3977,11 @@ struct StrackJob {
             while ((2 << lcc) <= wsR && (2 << lcc) * WA * 2 <= kStElems)
                 lcc++;
             const int Cx = 1 << lcx, Cc = 1 << lcc;
-            const int Rd = std::max(1, kStElems / (2 * WR)), nPd = (WA + Rd - 1) / Rd;
+            // 128 x 128 patches: the fixed-size passes of st_amp_large.h
+            const bool big = wsA == kAlWS && wsR == kAlWS && !staged_only();
+            const int Rd = std::max(1, kStElems / (2 * WR)), nPd = big ? kAlBlocks : (WA + Rd - 1) / Rd;
             const int Rf = kStElems / WR, nPf = (WA + Rf - 1) / Rf;
-            const int Rm = 2 * (kStElems / WR), nPm = (WA + Rm - 1) / Rm;
+            const int Rm = 2 * (kStElems / WR), nPm = big ? kAlMagBlocks : (WA + Rm - 1) / Rm;
             const size_t ldsX = (size_t)Cx * (Cx > 1 ? WA + 1 : WA) * sizeof(float2);
             const size_t ldsD = (size_t)2 * Rd * WR * sizeof(float2), ldsF = (size_t)Rf * WR * sizeof(float2);
             const size_t ldsC = (size_t)2 * Cc * (Cc > 1 ? WA + 1 : WA) * sizeof(float2);
@@ -4009,24 +4012,30 @@ struct StrackJob {
             for (int off = 0; off < nA; off += B) {
                 ctx->check_cancel();
                 const int nb = std::min(B, nA - off);
-                hipLaunchKernelGGL(k_amp_gather, dim3(nb), dim3(NT), 0, st, P, S, list, off, nb, large, A);
-                ctx->fft.rows(A.I, (long)2 * nb * wsA, wsR, -1, st);
-                hipLaunchKernelGGL(k_amp_colx, dim3((wsR + Cx - 1) / Cx, 2 * nb), dim3(NT), ldsX, st, A.I, nb, wsA, wsR,
-                                   A.az, A.state, A.F, lcx, PfsA, PiA, dA);
-                ctx->time_begin(kAmpDet);
-                hipLaunchKernelGGL(k_amp_rowdet, dim3(nPd, nb), dim3(NT), ldsD, st, P, A.F, nb, wsA, wsR, Rd, A.state,
-                                   (float *)A.S, A.dpart, PiR, dR);
-                ctx->time_end(kAmpDet);
-                hipLaunchKernelGGL(k_amp_stat, dim3(nb), dim3(64), 0, st, A.dpart, nPd, WA, WR, A.state, A.mean);
-                hipLaunchKernelGGL(k_amp_rowfwd, dim3(nPf, nb), dim3(NT), ldsF, st, (const float *)A.S, nb, WA, WR, Rf,
-                                   A.mean, A.state, A.F, A.ppart, PfR);
-                hipLaunchKernelGGL(k_amp_colx2, dim3((wsR + Cc - 1) / Cc, nb), dim3(NT), ldsC, st, A.F, WA, WR, A.state,
-                                   A.S, lcc, PfA, PiA, dA);
-                hipLaunchKernelGGL(k_amp_psum, dim3((nb + 127) / 128), dim3(128), 0, st, A.ppart, nPf, nb, WA, WR,
-                                   A.state, A.p);
+                if (big) {
+                    ctx->time_begin(kAmpDet);
+                    launch_amp_large(ctx, P, S, list + off, nb, large ? LA : 1, A);
+                    ctx->time_end(kAmpDet);
+                } else {
+                    hipLaunchKernelGGL(k_amp_gather, dim3(nb), dim3(NT), 0, st, P, S, list, off, nb, large, A);
+                    ctx->fft.rows(A.I, (long)2 * nb * wsA, wsR, -1, st);
+                    hipLaunchKernelGGL(k_amp_colx, dim3((wsR + Cx - 1) / Cx, 2 * nb), dim3(NT), ldsX, st, A.I, nb, wsA, wsR,
+                                       A.az, A.state, A.F, lcx, PfsA, PiA, dA);
+                    ctx->time_begin(kAmpDet);
+                    hipLaunchKernelGGL(k_amp_rowdet, dim3(nPd, nb), dim3(NT), ldsD, st, P, A.F, nb, wsA, wsR, Rd, A.state,
+                                       (float *)A.S, A.dpart, PiR, dR);
+                    ctx->time_end(kAmpDet);
+                    hipLaunchKernelGGL(k_amp_stat, dim3(nb), dim3(64), 0, st, A.dpart, nPd, WA, WR, A.state, A.mean);
+                    hipLaunchKernelGGL(k_amp_rowfwd, dim3(nPf, nb), dim3(NT), ldsF, st, (const float *)A.S, nb, WA, WR, Rf,
+                                       A.mean, A.state, A.F, A.ppart, PfR);
+                    hipLaunchKernelGGL(k_amp_colx2, dim3((wsR + Cc - 1) / Cc, nb), dim3(NT), ldsC, st, A.F, WA, WR, A.state,
+                                       A.S, lcc, PfA, PiA, dA);
+                    hipLaunchKernelGGL(k_amp_psum, dim3((nb + 127) / 128), dim3(128), 0, st, A.ppart, nPf, nb, WA, WR,
+                                       A.state, A.p);
+                    hipLaunchKernelGGL(k_amp_rowmag, dim3(nPm, nb), dim3(NT), ldsM, st, A.S, WA, WR, Rm, A.mag, A.part, PiR,
+                                       dR, A.state);
+                }
                 ctx->time_begin(kAmpPeak);
-                hipLaunchKernelGGL(k_amp_rowmag, dim3(nPm, nb), dim3(NT), ldsM, st, A.S, WA, WR, Rm, A.mag, A.part, PiR,
-                                   dR, A.state);
                 const GaussArg G{gauss ? 1 : 0, wsA, wsR, 1.0, 16.0, A.p};
                 if (gauss) {
                     hipLaunchKernelGGL(k_peak_merge<true>, dim3(nb), dim3(NT), 0, st, A.part, nPm, A.mag, WA, WR, 1,

@@ -25,9 +25,10 @@ def _pair(na, nr, seed, stype):
 
 
 @pytest.mark.parametrize("stype", [abi.ST_SAMPLE_C64, abi.ST_SAMPLE_CI16])
-@pytest.mark.parametrize("w,wa", [(16, 16), (32, 32), (64, 64), (32, 16), (24, 32)])
+@pytest.mark.parametrize("w,wa", [(16, 16), (32, 32), (64, 64), (32, 16), (24, 32), (64, 128)])
 def test_fused_tries_equal_staged_tries(device, monkeypatch, w, wa, stype):
-    na, nr = 20 * wa + 37, 18 * wa + 11
+    n = 20 if wa < 128 else 9
+    na, nr = n * wa + 37, (n - 2) * wa + 11
     a, b = _pair(na, nr, 7 + wa, stype)
     # the grid runs over the image's edges: some small and more doubled windows are out of bounds
     p = small_params(w, nr, na, step=wa - 3, wRa=wa, wAa=wa, noComplex=1, rStart=wa // 2, aStart=wa // 2,
@@ -40,7 +41,8 @@ def test_fused_tries_equal_staged_tries(device, monkeypatch, w, wa, stype):
         s = device.speckle_track(pid, p, diag=True)
     finally:
         device.release_pair(pid)
-    assert f.nAmp == s.nAmp > 0 and f.nAmpL == s.nAmpL > 0 and f.nFail == s.nFail > 0
+    assert f.nAmp == s.nAmp > 0 and f.nAmpL == s.nAmpL and f.nFail == s.nFail > 0
+    assert f.nAmpL > 0 or wa == 128
     for k in ("offR", "offA", "azd", "type"):
         assert np.array_equal(getattr(f, k), getattr(s, k)), k
     for k in ("peakI", "peakJ", "fineI", "fineJ", "sigRg", "sigAz", "peakGap", "fineGap"):
