@@ -29,12 +29,10 @@ namespace {
 
 constexpr float kNoData = -2.0e9f;
 constexpr int kMaxIter = 48;
-// The median kernels keep each wave's box values (range and azimuth) in
-// dynamic LDS sized for the box of the call, at most kCullLds bytes per
-// workgroup: box sides up to 45 (2025 cells; 4 waves x 2 x 4 B per cell).
+constexpr int kAhead = 3;  // fixpoint iterations launched before their change counts are read
+// Box sides of the median test (k_cull_iter's tile with its halo: 67 KB of LDS
+// at 45).
 constexpr int kMaxBox = 45;
-constexpr size_t kCullLds = 65536;
-constexpr int cull_box_cells(int bR, int bA) { return ((bR / 2) * 2 + 1) * ((bA / 2) * 2 + 1); }
 
 __device__ inline bool valid2(float r, float a)
 {
@@ -116,126 +114,205 @@ struct LsArg {
     double deltaT, dx, dy;
 };
 
-// Median test of one cell by one wavefront (cullSTData.c:73-122): the box
-// values are ranked by counting, the floor(n/2)-th smallest is the median
-// (selectForCull's k = n/2 on a 1-based list).  LS selects the Landsat
-// limits (cullLSData.c); maxA / maxR are then maxY / maxX.
+// Largest float not above m: d > m exactly when d > float_floor(m), for float d.
+__device__ inline float float_floor(double m)
+{
+    const float f = (float)m;
+    return (double)f > m ? nextafterf(f, -INFINITY) : f;
+}
+
+// The median test of cullSTData.c:73-122 without the median.  With n box
+// values the reference takes the k-th smallest m (k = n / 2, at least 1) and
+// culls the cell x when fl(x - m) leaves [-max, max].  fl(x - u) does not rise
+// with u, so the values u with fl(x - u) > max are the smallest ones: m is
+// among them exactly when there are at least k; and those with fl(x - u) <
+// -max are the largest: m is among them when there are at least n - k + 1.
+// Counting replaces the selection, and ties, infinities and a NaN x decide as
+// there (a comparison with NaN is false).
+struct MedianCount {
+    int n = 0, loR = 0, hiR = 0, loA = 0, hiA = 0;
+
+    // v: a box value pair, NaN when it takes no part
+    __device__ inline void add(float xR, float xA, float2 v, float maxR, float maxA)
+    {
+        const float dR = xR - v.x, dA = xA - v.y;
+        n += v.x == v.x;
+        loR += dR > maxR;
+        hiR += dR < -maxR;
+        loA += dA > maxA;
+        hiA += dA < -maxA;
+    }
+    __device__ inline bool off() const
+    {
+        const int k = n / 2 > 0 ? n / 2 : 1, m = n - k + 1;
+        return loR >= k || hiR >= m || loA >= k || hiA >= m;
+    }
+};
+
+// The slow-velocity limits of the Landsat variant, range then azimuth.
+__device__ inline float2 ls_slow_limits(const LsArg &L)
+{
+    const double m = 40.0 / 365. * L.deltaT;
+    double mX = m, mY = m;
+    mX /= L.dx;
+    mY /= L.dy;
+    mX = mX > 0.2 ? mX : 0.2;
+    mY = mY > 0.2 ? mY : 0.2;
+    return make_float2(float_floor(mX), float_floor(mY));
+}
+
+// The pair (r, a) of cell q, NaN when invalid or already culled.
+__device__ inline float2 box_value(const CullDev &D, int q, bool culled)
+{
+    const float r = D.R0[q], a = D.A0[q];
+    const float nan = __int_as_float(0x7fc00000);
+    return !culled && valid2(r, a) ? make_float2(r, a) : make_float2(nan, nan);
+}
+
+__device__ inline int wave_sum(int v)
+{
+    for (int o = 32; o > 0; o >>= 1)
+        v += __shfl_xor(v, o);
+    return v;
+}
+
+// Median test of one cell by one wavefront, lanes over the box; LS selects
+// the Landsat limits (cullLSData.c); maxA / maxR are then maxY / maxX.
 template <bool LS>
 __device__ inline bool cull_decide(const CullDev &D, int c, int bR, int bA, int nGood, float maxA, float maxR,
-                                   const uint8_t *earlier, float *lr, float *la, const LsArg &L)
+                                   const uint8_t *earlier, const LsArg &L)
 {
     const int lane = threadIdx.x & 63;
     const int i = c / D.nR, j = c - (c / D.nR) * D.nR;
     const int i1 = imax(0, i - bA / 2), i2 = imin(D.nA - 1, i + bA / 2);
     const int j1 = imax(0, j - bR / 2), j2 = imin(D.nR - 1, j + bR / 2);
     const int bw = j2 - j1 + 1, cnt = bw * (i2 - i1 + 1);
-    int ngood = 0;
-    bool anyFast = false;
-    for (int base = 0; base < cnt; base += 64) {
-        const int s = base + lane;
-        bool ok = false, fast = false;
-        float r = 0, a = 0;
-        if (s < cnt) {
-            const int q = (i1 + s / bw) * D.nR + j1 + s % bw;
-            const bool culled = q < c && earlier[q];
-            r = culled ? kNoData : D.R0[q];
-            a = culled ? kNoData : D.A0[q];
-            ok = valid2(r, a);
-            if constexpr (LS)
-                fast = ok && !(L.type[q] & L.slow);
+    auto value = [&](int s, int &q) {
+        q = (i1 + s / bw) * D.nR + j1 + s % bw;
+        return box_value(D, q, q < c && earlier[q]);
+    };
+    if constexpr (LS) {
+        bool fast = false;
+        for (int s = lane; s < cnt; s += 64) {
+            int q;
+            const float2 v = value(s, q);
+            fast |= v.x == v.x && !(L.type[q] & L.slow);
         }
-        if constexpr (LS)
-            anyFast = anyFast || __ballot(fast) != 0ull;
-        const unsigned long long m = __ballot(ok);
-        const int pos = ngood + __popcll(m & ((1ull << lane) - 1ull));
-        if (ok) {
-            lr[pos] = r;
-            la[pos] = a;
+        if (!__ballot(fast)) {
+            const float2 m = ls_slow_limits(L);
+            maxR = m.x;
+            maxA = m.y;
         }
-        ngood += __popcll(m);
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    if (ngood <= nGood)
+    const float xR = D.R0[c], xA = D.A0[c];
+    MedianCount M;
+    for (int s = lane; s < cnt; s += 64) {
+        int q;
+        M.add(xR, xA, value(s, q), maxR, maxA);
+    }
+    M.n = wave_sum(M.n);
+    M.loR = wave_sum(M.loR);
+    M.hiR = wave_sum(M.hiR);
+    M.loA = wave_sum(M.loA);
+    M.hiA = wave_sum(M.hiA);
+    if (M.n <= nGood)
         return true;
     if constexpr (LS) {
-        if (!((double)D.A0[c] > L.noData1))
+        if (!((double)xA > L.noData1))
             return true;
     }
-    int k = ngood / 2;
-    if (k == 0)
-        k = 1;
-    float medR = 0, medA = 0;
-    for (int base = 0; base < ngood; base += 64) {
-        const int s = base + lane;
-        bool isR = false, isA = false;
-        float vr = 0, va = 0;
-        if (s < ngood) {
-            vr = lr[s];
-            va = la[s];
-            int lessR = 0, eqR = 0, lessA = 0, eqA = 0;
-            for (int u = 0; u < ngood; u++) {
-                const float xr = lr[u], xa = la[u];
-                lessR += xr < vr;
-                eqR += xr == vr;
-                lessA += xa < va;
-                eqA += xa == va;
-            }
-            isR = lessR < k && k <= lessR + eqR;
-            isA = lessA < k && k <= lessA + eqA;
-        }
-        const unsigned long long mR = __ballot(isR), mA = __ballot(isA);
-        if (mR)
-            medR = __shfl(vr, __ffsll((long long)mR) - 1);
-        if (mA)
-            medA = __shfl(va, __ffsll((long long)mA) - 1);
-    }
-    const double diffA = (double)(D.A0[c] - medA);
-    const double diffR = (double)(D.R0[c] - medR);
-    if constexpr (LS) {
-        double mX = maxR, mY = maxA;
-        if (!anyFast) {
-            mX = 40.0 / 365. * L.deltaT;
-            mY = mX;
-            mX /= L.dx;
-            mY /= L.dy;
-            mX = mX > 0.2 ? mX : 0.2;
-            mY = mY > 0.2 ? mY : 0.2;
-        }
-        return fabs(diffA) > mY || fabs(diffR) > mX;
-    }
-    return fabs(diffA) > maxA || fabs(diffR) > maxR;
+    return M.off();
 }
 
+// One fixpoint iteration, a thread per cell: the tile of box values with its
+// halo in LDS twice, as they stand (E: culled cells of the previous iteration
+// out) and before any cull (N); a cell reads E for the cells before it in
+// raster order and N from itself on.  Bound: VALU, about 12 instructions per
+// box value (box 9 on 821 x 571 cells: 33 us per iteration; 1.13 ms with one
+// wave per cell ranking the box by counting).
+constexpr int kTileR = 32, kTileA = 8;  // 256 threads
+constexpr size_t cull_tile_bytes(int bR, int bA, bool ls)
+{
+    return (size_t)(kTileR + bR / 2 * 2) * (kTileA + bA / 2 * 2) * (2 * sizeof(float2) + (ls ? 1 : 0));
+}
 template <bool LS>
 __global__ void __launch_bounds__(256) k_cull_iter(CullDev D, int bR, int bA, int nGood, float maxA, float maxR,
-                                                   LsArg L)
+                                                   LsArg L, int slot)
 {
-    extern __shared__ float cull_lds[];  // per wave: range values, then azimuth values
-    const int w = threadIdx.x >> 6, cells = cull_box_cells(bR, bA);
-    const int c = blockIdx.x * 4 + w;
-    if (c >= D.nR * D.nA)
-        return;
-    float *lr = cull_lds + (size_t)w * 2 * cells, *la = lr + cells;
-    const bool cull = cull_decide<LS>(D, c, bR, bA, nGood, maxA, maxR, D.cPrev, lr, la, L);
-    if ((threadIdx.x & 63) == 0) {
-        D.cNew[c] = cull ? 1 : 0;
-        if ((D.cPrev[c] != 0) != cull)
-            atomicAdd(&D.counters[0], 1);
+    extern __shared__ float2 cull_lds[];
+    const int hR = bR / 2, hA = bA / 2, tw = kTileR + 2 * hR, cells = tw * (kTileA + 2 * hA);
+    float2 *E = cull_lds, *N = cull_lds + cells;
+    uint8_t *fastB = (uint8_t *)(cull_lds + 2 * cells);
+    const int nbx = (D.nR + kTileR - 1) / kTileR, t = threadIdx.x;
+    const int i0 = (int)blockIdx.x / nbx * kTileA, j0 = (int)blockIdx.x % nbx * kTileR;
+    for (int e = t; e < cells; e += 256) {
+        const int ii = i0 - hA + e / tw, jj = j0 - hR + e % tw;
+        const float nan = __int_as_float(0x7fc00000);
+        float2 n = make_float2(nan, nan), v = n;
+        bool fast = false;
+        if (ii >= 0 && ii < D.nA && jj >= 0 && jj < D.nR) {
+            const int q = ii * D.nR + jj;
+            n = box_value(D, q, false);
+            v = D.cPrev[q] ? v : n;
+            if constexpr (LS)
+                fast = !(L.type[q] & L.slow);
+        }
+        N[e] = n;
+        E[e] = v;
+        if constexpr (LS)
+            fastB[e] = fast;
     }
+    __syncthreads();
+    const int ti = t / kTileR, tj = t % kTileR, i = i0 + ti, j = j0 + tj;
+    bool changed = false;
+    if (i < D.nA && j < D.nR) {
+        const int c = i * D.nR + j, bw = 2 * hR + 1, at = ti * tw + tj;
+        if constexpr (LS) {
+            bool fast = false;
+            for (int a = 0; a <= 2 * hA; a++)
+                for (int r = 0; r < bw; r++) {
+                    const int e = at + a * tw + r;
+                    const float x = (a < hA || (a == hA && r < hR) ? E[e] : N[e]).x;
+                    fast |= x == x && fastB[e];
+                }
+            if (!fast) {
+                const float2 m = ls_slow_limits(L);
+                maxR = m.x;
+                maxA = m.y;
+            }
+        }
+        const float xR = D.R0[c], xA = D.A0[c];
+        MedianCount M;
+        for (int a = 0; a < hA; a++)
+#pragma unroll 3
+            for (int r = 0; r < bw; r++)
+                M.add(xR, xA, E[at + a * tw + r], maxR, maxA);
+        for (int r = 0; r < hR; r++)
+            M.add(xR, xA, E[at + hA * tw + r], maxR, maxA);
+        for (int r = hR; r < bw; r++)
+            M.add(xR, xA, N[at + hA * tw + r], maxR, maxA);
+        for (int a = hA + 1; a <= 2 * hA; a++)
+#pragma unroll 3
+            for (int r = 0; r < bw; r++)
+                M.add(xR, xA, N[at + a * tw + r], maxR, maxA);
+        bool cull = M.n <= nGood || M.off();
+        if constexpr (LS)
+            cull = cull || !((double)xA > L.noData1);
+        D.cNew[c] = cull ? 1 : 0;
+        changed = (D.cPrev[c] != 0) != cull;
+    }
+    const unsigned long long m = __ballot(changed);
+    if (m && (t & 63) == 0)
+        atomicAdd(&D.counters[slot], __popcll(m));
 }
 
-// Exact sequential order for the leftover case: one workgroup (up to 16
-// waves, fewer for large boxes) sweeps the wavefront steps, one wave per
-// cell of a step.
+// Exact sequential order for the leftover case: one workgroup sweeps the
+// wavefront steps, one wave per cell of a step.
 template <bool LS>
 __global__ void __launch_bounds__(1024) k_cull_wavefront(CullDev D, int bR, int bA, int nGood, float maxA, float maxR,
                                                          LsArg L)
 {
-    extern __shared__ float cull_lds[];
-    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6, cells = cull_box_cells(bR, bA);
-    float *lr = cull_lds + (size_t)w * 2 * cells, *la = lr + cells;
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int s = bR / 2 + 1;
     const int steps = (D.nA - 1) * s + D.nR;
     for (int T = 0; T < steps; T++) {
@@ -244,7 +321,7 @@ __global__ void __launch_bounds__(1024) k_cull_wavefront(CullDev D, int bR, int 
         for (int i = iLo + w; i <= iHi; i += nw) {
             const int j = T - i * s;
             const int c = i * D.nR + j;
-            const bool cull = cull_decide<LS>(D, c, bR, bA, nGood, maxA, maxR, D.cNew, lr, la, L);
+            const bool cull = cull_decide<LS>(D, c, bR, bA, nGood, maxA, maxR, D.cNew, L);
             if ((threadIdx.x & 63) == 0)
                 D.cNew[c] = cull ? 1 : 0;
         }
@@ -255,42 +332,65 @@ __global__ void __launch_bounds__(1024) k_cull_wavefront(CullDev D, int bR, int 
 __global__ void k_cull_apply(CullDev D)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= D.nR * D.nA)
-        return;
-    if (D.cNew[c]) {
-        D.offR[c] = kNoData;
-        D.offA[c] = kNoData;
-        atomicAdd(&D.counters[1], 1);
-    } else {
-        D.offR[c] = D.R0[c];
-        D.offA[c] = D.A0[c];
+    const bool in = c < D.nR * D.nA, cull = in && D.cNew[c];
+    if (in) {
+        D.offR[c] = cull ? kNoData : D.R0[c];
+        D.offA[c] = cull ? kNoData : D.A0[c];
     }
+    const unsigned long long m = __ballot(cull);
+    if (m && (threadIdx.x & 63) == 0)
+        atomicAdd(&D.counters[1], __popcll(m));
 }
 
-// cullStats (cullStats.c:19-144) with the plane fit done by a one-sided
-// Jacobi SVD whose rotated columns are recomputed from the box rows (the
-// oracle follows the same arithmetic).  Sweeps stop at column-pair cosines
-// below 1e-13, just above the rounding floor of the 81-row sums.
-__device__ void lsq3(double c0, const CullDev &D, int i1, int i2, int j1, int j2, bool useR, double x[3])
+// The plane fit of cullStats: least squares y ~ A x over the box's n good
+// points, A's rows (c0, ii, jj), singular values below 1e-5 of the largest
+// dropped (svdfit's rule).  A = B T with B's rows (1, di, dj), di = ii - i and
+// dj = jj - j, and T = [c0 i j; 0 1 0; 0 0 1]; B's Gram matrix holds small
+// integers, so its Cholesky factor L is exact to a rounding and A = Q (L^T T)
+// with orthonormal Q: the one-sided Jacobi SVD of A's columns is that of the
+// 3 x 3 matrix L^T T, and u_k . y is (L^T T v_k) . (Q^T y).  The sweeps run
+// over three rows instead of the 81 of the box; they stop at column-pair
+// cosines below 1e-13.
+struct BoxGram {
+    double l11, l21, l31, l22, l32, l33;
+
+    __device__ inline void factor(int n, int si, int sj, int sii, int sij, int sjj)
+    {
+        // every numerator is an exact integer (n <= 81, |di|, |dj| <= 4)
+        const double dn = (double)n;
+        const double pii = (double)(n * sii - si * si), pij = (double)(n * sij - si * sj), pjj = (double)(n * sjj - sj * sj);
+        l11 = sqrt(dn);
+        l21 = (double)si / l11;
+        l31 = (double)sj / l11;
+        l22 = sqrt(pii / dn);
+        l32 = pii > 0.0 ? pij / (dn * l22) : 0.0;
+        l33 = pii > 0.0 ? sqrt((pii * pjj - pij * pij) / (dn * pii)) : sqrt(pjj / dn);
+    }
+};
+
+// b: B^T y.
+__device__ inline void lsq3(double c0, double i, double j, const BoxGram &G, const double b[3], double x[3])
 {
+    const double R[3][3] = {{G.l11 * c0, G.l11 * i + G.l21, G.l11 * j + G.l31}, {0.0, G.l22, G.l32}, {0.0, 0.0, G.l33}};
+    const double z0 = b[0] / G.l11;
+    const double z1 = G.l22 > 0.0 ? (b[1] - G.l21 * z0) / G.l22 : 0.0;
+    const double z2 = G.l33 > 0.0 ? (b[2] - G.l31 * z0 - G.l32 * z1) / G.l33 : 0.0;
     double V[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
     for (int sweep = 0; sweep < 30; sweep++) {
         double off = 0.0;
+#pragma unroll
         for (int p = 0; p < 2; p++)
+#pragma unroll
             for (int q = p + 1; q < 3; q++) {
                 double alpha = 0, beta = 0, gamma = 0;
-                for (int ii = i1; ii <= i2; ii++)
-                    for (int jj = j1; jj <= j2; jj++) {
-                        const int o = ii * D.nR + jj;
-                        if (!valid2(D.offR[o], D.offA[o]))
-                            continue;
-                        const double a0 = c0, a1 = (double)ii, a2 = (double)jj;
-                        const double up = a0 * V[0 * 3 + p] + a1 * V[1 * 3 + p] + a2 * V[2 * 3 + p];
-                        const double uq = a0 * V[0 * 3 + q] + a1 * V[1 * 3 + q] + a2 * V[2 * 3 + q];
-                        alpha += up * up;
-                        beta += uq * uq;
-                        gamma += up * uq;
-                    }
+#pragma unroll
+                for (int r = 0; r < 3; r++) {
+                    const double up = R[r][0] * V[0 * 3 + p] + R[r][1] * V[1 * 3 + p] + R[r][2] * V[2 * 3 + p];
+                    const double uq = R[r][0] * V[0 * 3 + q] + R[r][1] * V[1 * 3 + q] + R[r][2] * V[2 * 3 + q];
+                    alpha += up * up;
+                    beta += uq * uq;
+                    gamma += up * uq;
+                }
                 if (gamma == 0.0)
                     continue;
                 const double conv = fabs(gamma) / sqrt(alpha * beta);
@@ -301,6 +401,7 @@ __device__ void lsq3(double c0, const CullDev &D, int i1, int i2, int j1, int j2
                 const double zeta = (beta - alpha) / (2.0 * gamma);
                 const double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
                 const double c = 1.0 / sqrt(1.0 + t * t), s = c * t;
+#pragma unroll
                 for (int r = 0; r < 3; r++) {
                     const double vp = V[r * 3 + p], vq = V[r * 3 + q];
                     V[r * 3 + p] = c * vp - s * vq;
@@ -310,88 +411,113 @@ __device__ void lsq3(double c0, const CullDev &D, int i1, int i2, int j1, int j2
         if (off < 1e-13)
             break;
     }
-    double w2[3] = {0, 0, 0}, uy[3] = {0, 0, 0};
-    for (int ii = i1; ii <= i2; ii++)
-        for (int jj = j1; jj <= j2; jj++) {
-            const int o = ii * D.nR + jj;
-            if (!valid2(D.offR[o], D.offA[o]))
-                continue;
-            const double yv = useR ? (double)D.offR[o] : (double)D.offA[o];
-            const double a0 = c0, a1 = (double)ii, a2 = (double)jj;
-            for (int k = 0; k < 3; k++) {
-                const double u = a0 * V[0 * 3 + k] + a1 * V[1 * 3 + k] + a2 * V[2 * 3 + k];
-                w2[k] += u * u;
-                uy[k] += u * yv;
-            }
-        }
-    double w[3], wmax = 0;
+    double w2[3], uy[3], w[3], wmax = 0;
+#pragma unroll
     for (int k = 0; k < 3; k++) {
+        w2[k] = uy[k] = 0;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const double u = R[r][0] * V[0 * 3 + k] + R[r][1] * V[1 * 3 + k] + R[r][2] * V[2 * 3 + k];
+            w2[k] += u * u;
+            uy[k] += u * (r == 0 ? z0 : r == 1 ? z1 : z2);
+        }
         w[k] = sqrt(w2[k]);
         if (w[k] > wmax)
             wmax = w[k];
     }
     const double thresh = 1.0e-5 * wmax;
     double coef[3];
+#pragma unroll
     for (int k = 0; k < 3; k++)
         coef[k] = (w[k] < thresh || w[k] == 0.0) ? 0.0 : uy[k] / w2[k];
+#pragma unroll
     for (int r = 0; r < 3; r++)
         x[r] = V[r * 3 + 0] * coef[0] + V[r * 3 + 1] * coef[1] + V[r * 3 + 2] * coef[2];
 }
 
-// addQuant: cullLSStats adds the quantisation variance `quant` before the
-// square root (cullLSStats.c:144-146).
-__global__ void k_cull_stats(CullDev D, int addQuant, double quant)
+// cullStats (cullStats.c:19-144), a thread per cell, the 9 x 9 boxes from an
+// LDS tile.  Bound: FP64 VALU (two passes over 81 box values and the 3 x 3
+// sweeps).  addQuant: cullLSStats adds the quantisation variance `quant`
+// before the square root (cullLSStats.c:144-146).
+__global__ void __launch_bounds__(256) k_cull_stats(CullDev D, int addQuant, double quant)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= D.nR * D.nA)
+    constexpr int b = 9, h = b / 2, tw = kTileR + 2 * h, cells = tw * (kTileA + 2 * h);
+    __shared__ float2 tile[cells];  // NaN: no good value
+    const int nbx = (D.nR + kTileR - 1) / kTileR, t = threadIdx.x;
+    const int i0 = (int)blockIdx.x / nbx * kTileA, j0 = (int)blockIdx.x % nbx * kTileR;
+    for (int e = t; e < cells; e += 256) {
+        const int ii = i0 - h + e / tw, jj = j0 - h + e % tw;
+        const float nan = __int_as_float(0x7fc00000);
+        float2 v = make_float2(nan, nan);
+        if (ii >= 0 && ii < D.nA && jj >= 0 && jj < D.nR) {
+            const int q = ii * D.nR + jj;
+            const float r = D.offR[q], a = D.offA[q];
+            if (valid2(r, a))
+                v = make_float2(r, a);
+        }
+        tile[e] = v;
+    }
+    __syncthreads();
+    const int ti = t / kTileR, tj = t % kTileR, i = i0 + ti, j = j0 + tj, at = ti * tw + tj;
+    if (i >= D.nA || j >= D.nR)
         return;
-    const int b = 9;
-    const int i = c / D.nR, j = c - (c / D.nR) * D.nR;
-    const int i1 = imax(0, i - b / 2), i2 = imin(D.nA - 1, i + b / 2);
-    const int j1 = imax(0, j - b / 2), j2 = imin(D.nR - 1, j + b / 2);
-    int ngood = 0;
-    double meanA = 0.0, meanR = 0.0;
-    for (int ii = i1; ii <= i2; ii++)
-        for (int jj = j1; jj <= j2; jj++) {
-            const int o = ii * D.nR + jj;
-            if (valid2(D.offR[o], D.offA[o])) {
-                ngood++;
-                meanA += D.offA[o];
-                meanR += D.offR[o];
+    const int c = i * D.nR + j;
+    int n = 0, si = 0, sj = 0, sii = 0, sij = 0, sjj = 0;
+    double meanA = 0.0, meanR = 0.0, bR[3] = {0, 0, 0}, bA[3] = {0, 0, 0};
+    for (int di = -h; di <= h; di++)
+#pragma unroll
+        for (int dj = -h; dj <= h; dj++) {
+            const float2 v = tile[at + (di + h) * tw + dj + h];
+            if (v.x == v.x) {
+                n++;
+                si += di;
+                sj += dj;
+                sii += di * di;
+                sij += di * dj;
+                sjj += dj * dj;
+                meanA += v.y;
+                meanR += v.x;
+                bR[1] += (double)di * v.x;
+                bR[2] += (double)dj * v.x;
+                bA[1] += (double)di * v.y;
+                bA[2] += (double)dj * v.y;
             }
         }
-    meanA /= (double)ngood;
-    meanR /= (double)ngood;
-    if (!(ngood > 8 && D.offR[c] > (float)(1 - ST_LARGEINT))) {
+    if (!(n > 8 && D.offR[c] > (float)(1 - ST_LARGEINT))) {
         D.sigmaA[c] = kNoData;
         D.sigmaR[c] = kNoData;
         return;
     }
+    bR[0] = meanR;
+    bA[0] = meanA;
+    meanA /= (double)n;
+    meanR /= (double)n;
+    BoxGram G;
+    G.factor(n, si, sj, sii, sij, sjj);
     double aR[3], aA[3];
-    lsq3((double)(float)meanR, D, i1, i2, j1, j2, true, aR);
-    lsq3((double)(float)meanA, D, i1, i2, j1, j2, false, aA);
+    lsq3((double)(float)meanR, (double)i, (double)j, G, bR, aR);
+    lsq3((double)(float)meanA, (double)i, (double)j, G, bA, aA);
     aR[0] *= meanR;
     aA[0] *= meanA;
-    int ng = 0;
     double mA = 0.0, mR = 0.0, varR = 0.0, varA = 0.0;
-    for (int ii = i1; ii <= i2; ii++)
-        for (int jj = j1; jj <= j2; jj++) {
-            const int o = ii * D.nR + jj;
-            if (valid2(D.offR[o], D.offA[o])) {
-                ng++;
-                float oR = D.offR[o], oA = D.offA[o];
-                oR = (float)(oR - (aR[0] + aR[1] * (float)ii + aR[2] * (float)jj));
-                oA = (float)(oA - (aA[0] + aA[1] * (float)ii + aA[2] * (float)jj));
+    for (int di = -h; di <= h; di++)
+#pragma unroll
+        for (int dj = -h; dj <= h; dj++) {
+            const float2 v = tile[at + (di + h) * tw + dj + h];
+            if (v.x == v.x) {
+                const float ii = (float)(i + di), jj = (float)(j + dj);
+                const float oR = (float)(v.x - (aR[0] + aR[1] * ii + aR[2] * jj));
+                const float oA = (float)(v.y - (aA[0] + aA[1] * ii + aA[2] * jj));
                 mA += oA;
                 mR += oR;
                 varA += oA * oA;
                 varR += oR * oR;
             }
         }
-    float sA = (float)(varA / (float)(ng - 3));
-    float sR = (float)(varR / (float)(ng - 3));
-    sA = (float)(sA - mA * mA / (float)((ng - 3) * ng));
-    sR = (float)(sR - mR * mR / (float)((ng - 3) * ng));
+    float sA = (float)(varA / (float)(n - 3));
+    float sR = (float)(varR / (float)(n - 3));
+    sA = (float)(sA - mA * mA / (float)((n - 3) * n));
+    sR = (float)(sR - mR * mR / (float)((n - 3) * n));
     sA = (float)(0.00001 > sA ? 0.00001 : sA);
     sR = (float)(0.00001 > sR ? 0.00001 : sR);
     if (addQuant) {
@@ -526,32 +652,38 @@ __device__ inline void uf_unite(int *par, int a, int b)
     }
 }
 
-// Each valid cell starts linked to its left neighbour when that is valid,
-// else to the one above, so a row run is one chain before any merge.
+// Each valid cell starts linked to the first cell of its row run (within the
+// 64 cells of its wave; a run that comes in from the wave before is linked on
+// at the wave's first cell), and a run's first cell to the one above it when
+// that is valid.
 __global__ void k_isl_init(CullDev D)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= D.nR * D.nA)
+    const int c = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+    const bool in = c < D.nR * D.nA, v = in && isl_valid(D, c);
+    const bool start = v && !(c % D.nR > 0 && isl_valid(D, c - 1));
+    const unsigned long long m = __ballot(start) & ((2ull << lane) - 1ull);
+    if (!in)
         return;
     int p = c;
-    if (isl_valid(D, c)) {
-        const int j = c % D.nR;
-        if (j > 0 && isl_valid(D, c - 1))
-            p = c - 1;
-        else if (c >= D.nR && isl_valid(D, c - D.nR))
+    if (start) {
+        if (c >= D.nR && isl_valid(D, c - D.nR))
             p = c - D.nR;
+    } else if (v) {
+        p = m ? c - lane + 63 - __clzll((long long)m) : lane ? c - lane : c - 1;
     }
     D.parent[c] = p;
 }
 
-// The only edge the initial links leave out: up, when left was taken.
+// The edges the initial links leave out: up, from a cell that is not the
+// first of its run; and of those only where the run above begins, or the cell
+// to the left would have made the same join.
 __global__ void k_isl_merge(CullDev D)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= D.nR * D.nA || c < D.nR || !isl_valid(D, c))
         return;
     const int j = c % D.nR;
-    if (j > 0 && isl_valid(D, c - 1) && isl_valid(D, c - D.nR))
+    if (j > 0 && isl_valid(D, c - 1) && isl_valid(D, c - D.nR) && !isl_valid(D, c - D.nR - 1))
         uf_unite(D.parent, c, c - D.nR);
 }
 
@@ -573,7 +705,9 @@ __global__ void k_isl_bbox(CullDev D)
     for (int o = 32; o > 0; o >>= 1)
         rmax = max(rmax, __shfl_xor(rmax, o));
     const int lane = threadIdx.x & 63;
-    if (lane == 0 && rmax >= 0)
+    // (atomics only where they would change the value: every wave of the large
+    // component meets the same five words)
+    if (lane == 0 && rmax > uf_ld(D.counters, 2))
         atomicMax(&D.counters[2], rmax);
     unsigned long long pending = __ballot(v);
     while (pending) {
@@ -589,10 +723,14 @@ __global__ void k_isl_bbox(CullDev D)
             imax = max(imax, __shfl_xor(imax, o));
         }
         if (lane == leader) {
-            atomicMin(&D.bbox[4 * rl + 0], jmin);
-            atomicMax(&D.bbox[4 * rl + 1], jmax);
-            atomicMin(&D.bbox[4 * rl + 2], imin);
-            atomicMax(&D.bbox[4 * rl + 3], imax);
+            if (jmin < uf_ld(D.bbox, 4 * rl + 0))
+                atomicMin(&D.bbox[4 * rl + 0], jmin);
+            if (jmax > uf_ld(D.bbox, 4 * rl + 1))
+                atomicMax(&D.bbox[4 * rl + 1], jmax);
+            if (imin < uf_ld(D.bbox, 4 * rl + 2))
+                atomicMin(&D.bbox[4 * rl + 2], imin);
+            if (imax > uf_ld(D.bbox, 4 * rl + 3))
+                atomicMax(&D.bbox[4 * rl + 3], imax);
         }
         pending &= ~__ballot(mine);
     }
@@ -738,6 +876,8 @@ struct CullRun {
         if (h)
             ST_HIP(hipMemcpyAsync(h, d, cnt * sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
     }
+    // one workgroup per kTileR x kTileA cells
+    dim3 tiles() const { return dim3((unsigned)((D.nR + kTileR - 1) / kTileR) * (unsigned)((D.nA + kTileA - 1) / kTileA)); }
     int counter(int k)
     {
         int v = 0;
@@ -760,25 +900,28 @@ struct CullRun {
         ST_REQUIRE(bR >= 1 && bA >= 1 && (bR / 2) * 2 + 1 <= kMaxBox && (bA / 2) * 2 + 1 <= kMaxBox,
                    ST_ERR_UNSUPPORTED, "box sizes above 45");
         hipStream_t st = ctx->stream;
-        const size_t perWave = 2 * sizeof(float) * (size_t)cull_box_cells(bR, bA);
-        const int wfWaves = (int)std::min<size_t>(16, kCullLds / perWave);
         bool settled = false;
         const int maxIter = max_iterations();
-        for (int it = 0; it < maxIter; it++) {
-            ST_HIP(hipMemsetAsync(D.counters, 0, sizeof(int), st));
-            hipLaunchKernelGGL(k_cull_iter<LS>, dim3((n + 3) / 4), dim3(256), 4 * perWave, st, D, bR, bA, nGood, maxA,
-                               maxR, L);
-            ST_HIP(hipGetLastError());
-            std::swap(D.cPrev, D.cNew);
-            if (counter(0) == 0) {
-                settled = true;
-                break;
+        // kAhead iterations per look at their change counts (counters 5 ..): a
+        // pass settles in two or three, and iterations after that change nothing
+        for (int it = 0; it < maxIter && !settled;) {
+            const int ahead = std::min(kAhead, maxIter - it);
+            ST_HIP(hipMemsetAsync(D.counters + 5, 0, kAhead * sizeof(int), st));
+            for (int k = 0; k < ahead; k++, it++) {
+                hipLaunchKernelGGL(k_cull_iter<LS>, tiles(), dim3(256), cull_tile_bytes(bR, bA, LS), st, D, bR, bA, nGood,
+                                   maxA, maxR, L, 5 + k);
+                std::swap(D.cPrev, D.cNew);
             }
+            ST_HIP(hipGetLastError());
+            int changed[kAhead];
+            ST_HIP(hipMemcpyAsync(changed, D.counters + 5, sizeof(changed), hipMemcpyDeviceToHost, st));
+            ST_HIP(hipStreamSynchronize(st));
+            for (int k = 0; k < ahead; k++)
+                settled = settled || changed[k] == 0;
         }
         std::swap(D.cPrev, D.cNew);  // cNew holds the last decisions
         if (!settled)
-            hipLaunchKernelGGL(k_cull_wavefront<LS>, dim3(1), dim3(64 * wfWaves), wfWaves * perWave, st, D, bR, bA,
-                               nGood, maxA, maxR, L);
+            hipLaunchKernelGGL(k_cull_wavefront<LS>, dim3(1), dim3(1024), 0, st, D, bR, bA, nGood, maxA, maxR, L);
         ST_HIP(hipMemsetAsync(D.counters + 1, 0, sizeof(int), st));
         hipLaunchKernelGGL(k_cull_apply, dim3(nb(n)), dim3(256), 0, st, D);
         ST_HIP(hipGetLastError());
@@ -787,7 +930,7 @@ struct CullRun {
     void stats()
     {
         cp->bR = cp->bA = 9;  // cullStats.c:38-39
-        hipLaunchKernelGGL(k_cull_stats, dim3(nb(n)), dim3(256), 0, ctx->stream, D, 0, 0.0);
+        hipLaunchKernelGGL(k_cull_stats, tiles(), dim3(256), 0, ctx->stream, D, 0, 0.0);
         ST_HIP(hipGetLastError());
     }
     void smooth()
@@ -1037,7 +1180,7 @@ struct CullLSRun {
         ST_REQUIRE(cp->nover > 0, ST_ERR_ARG, "nover");
         cp->bR = cp->bA = 9;  // cullLSStats.c:39-40
         const double q = ((1.0 / cp->nover) * (1.0 / cp->nover)) / 12.;
-        hipLaunchKernelGGL(k_cull_stats, dim3(nb(R.n)), dim3(256), 0, R.ctx->stream, R.D, 1, q);
+        hipLaunchKernelGGL(k_cull_stats, R.tiles(), dim3(256), 0, R.ctx->stream, R.D, 1, q);
         ST_HIP(hipGetLastError());
     }
     void ls_smooth()
