@@ -29,6 +29,7 @@ namespace {
 
 constexpr float kNoData = -2.0e9f;
 constexpr int kMaxIter = 48;
+constexpr int kCullCount = 8, kCullSlots = 8;  // words of CullDev::counters that count the culled cells
 constexpr int kAhead = 3;  // fixpoint iterations launched before their change counts are read
 // Box sides of the median test (k_cull_iter's tile with its halo: 67 KB of LDS
 // at 45).
@@ -47,7 +48,7 @@ struct CullDev {
     float *offRS, *offAS, *sigmaR, *sigmaA;
     float *R0, *A0;       // state at the start of a cullSTData pass
     uint8_t *cPrev, *cNew; // cull decisions of the pass
-    int *counters;        // [0] changed, [1] nCulled, [2] max root, ...
+    int *counters;        // [2] max root, [3] good cells, [4] cells with data, [5 ..] changes per iteration, [8 ..] culled cells
     int *parent, *root, *bbox;   // islands
 };
 
@@ -228,7 +229,7 @@ __device__ inline bool cull_decide(const CullDev &D, int c, int bR, int bA, int 
 // halo in LDS twice, as they stand (E: culled cells of the previous iteration
 // out) and before any cull (N); a cell reads E for the cells before it in
 // raster order and N from itself on.  Bound: VALU, about 12 instructions per
-// box value (box 9 on 821 x 571 cells: 33 us per iteration; 1.13 ms with one
+// box value (box 9 on 821 x 571 cells: 45 us per iteration; 1.13 ms with one
 // wave per cell ranking the box by counting).
 constexpr int kTileR = 32, kTileA = 8;  // 256 threads
 constexpr size_t cull_tile_bytes(int bR, int bA, bool ls)
@@ -338,8 +339,17 @@ __global__ void k_cull_apply(CullDev D)
         D.offA[c] = cull ? kNoData : D.A0[c];
     }
     const unsigned long long m = __ballot(cull);
-    if (m && (threadIdx.x & 63) == 0)
-        atomicAdd(&D.counters[1], __popcll(m));
+    __shared__ int part[4];
+    if ((threadIdx.x & 63) == 0)
+        part[threadIdx.x >> 6] = __popcll(m);
+    __syncthreads();
+    // spread over kCullSlots words: one word takes some 12 ns per atomic, and
+    // a whole scene has thousands of workgroups
+    if (threadIdx.x == 0) {
+        const int k = part[0] + part[1] + part[2] + part[3];
+        if (k)
+            atomicAdd(&D.counters[kCullCount + blockIdx.x % kCullSlots], k);
+    }
 }
 
 // The plane fit of cullStats: least squares y ~ A x over the box's n good
@@ -902,30 +912,36 @@ struct CullRun {
         hipStream_t st = ctx->stream;
         bool settled = false;
         const int maxIter = max_iterations();
-        // kAhead iterations per look at their change counts (counters 5 ..): a
-        // pass settles in two or three, and iterations after that change nothing
-        for (int it = 0; it < maxIter && !settled;) {
+        int got[kCullCount + kCullSlots - 5];  // counters 5 ..
+        // kAhead iterations and the culls applied per look at the change counts:
+        // a pass settles in two or three, iterations after that change nothing,
+        // and applying is repeated if it had not settled
+        for (int it = 0; !settled;) {
             const int ahead = std::min(kAhead, maxIter - it);
-            ST_HIP(hipMemsetAsync(D.counters + 5, 0, kAhead * sizeof(int), st));
+            ST_HIP(hipMemsetAsync(D.counters + 5, 0, sizeof(got), st));
             for (int k = 0; k < ahead; k++, it++) {
                 hipLaunchKernelGGL(k_cull_iter<LS>, tiles(), dim3(256), cull_tile_bytes(bR, bA, LS), st, D, bR, bA, nGood,
                                    maxA, maxR, L, 5 + k);
                 std::swap(D.cPrev, D.cNew);
             }
+            std::swap(D.cPrev, D.cNew);  // cNew holds the last decisions
+            if (ahead <= 0) {
+                hipLaunchKernelGGL(k_cull_wavefront<LS>, dim3(1), dim3(1024), 0, st, D, bR, bA, nGood, maxA, maxR, L);
+                settled = true;
+            }
+            hipLaunchKernelGGL(k_cull_apply, dim3(nb(n)), dim3(256), 0, st, D);
             ST_HIP(hipGetLastError());
-            int changed[kAhead];
-            ST_HIP(hipMemcpyAsync(changed, D.counters + 5, sizeof(changed), hipMemcpyDeviceToHost, st));
+            ST_HIP(hipMemcpyAsync(got, D.counters + 5, sizeof(got), hipMemcpyDeviceToHost, st));
             ST_HIP(hipStreamSynchronize(st));
             for (int k = 0; k < ahead; k++)
-                settled = settled || changed[k] == 0;
+                settled = settled || got[k] == 0;
+            if (!settled)
+                std::swap(D.cPrev, D.cNew);
         }
-        std::swap(D.cPrev, D.cNew);  // cNew holds the last decisions
-        if (!settled)
-            hipLaunchKernelGGL(k_cull_wavefront<LS>, dim3(1), dim3(1024), 0, st, D, bR, bA, nGood, maxA, maxR, L);
-        ST_HIP(hipMemsetAsync(D.counters + 1, 0, sizeof(int), st));
-        hipLaunchKernelGGL(k_cull_apply, dim3(nb(n)), dim3(256), 0, st, D);
-        ST_HIP(hipGetLastError());
-        return counter(1);
+        int culled = 0;
+        for (int k = 0; k < kCullSlots; k++)
+            culled += got[kCullCount - 5 + k];
+        return culled;
     }
     void stats()
     {
@@ -1047,13 +1063,28 @@ extern "C" int st_cull_islands(st_ctx *c, st_cull_params *cp)
 namespace {
 
 // cullst's order on host grids: upload, cullSTData x3, cullStats,
-// cullSmooth, cullIslands, download.
-void cull_chain_host(st_ctx *c, st_cull_params *cp, CullRun &R)
+// cullSmooth, cullIslands, download.  staged: through the context's pinned
+// buffer, one copy each way over the run of grids alloc() carves (copies from
+// and to pageable memory go through the driver's own staging, one grid after
+// another).
+void cull_chain_host(st_ctx *c, st_cull_params *cp, CullRun &R, bool staged)
 {
-    R.put(R.D.offR, cp->offR, R.n);
-    R.put(R.D.offA, cp->offA, R.n);
-    R.put(R.D.corr, cp->corr, R.n);
-    R.put(R.D.type, cp->type, R.n);
+    const CullDev &D = R.D;
+    const size_t f4 = (size_t)R.n * sizeof(float);
+    char *const dev = (char *)D.offR;  // the first of the grids
+    const size_t in = (size_t)((char *)D.type - dev) + R.n, all = (size_t)((char *)D.sigmaA - dev) + f4;
+    char *stg = staged ? (char *)c->pinned_reserve(all) : nullptr;
+    auto at = [&](const void *d) { return stg + ((const char *)d - dev); };
+    if (staged) {
+        parallel_copy({{at(D.offR), cp->offR, f4}, {at(D.offA), cp->offA, f4}, {at(D.corr), cp->corr, f4},
+                       {at(D.type), cp->type, (size_t)R.n}});
+        ST_HIP(hipMemcpyAsync(dev, stg, in, hipMemcpyHostToDevice, c->stream));
+    } else {
+        R.put(D.offR, cp->offR, R.n);
+        R.put(D.offA, cp->offA, R.n);
+        R.put(D.corr, cp->corr, R.n);
+        R.put(D.type, cp->type, R.n);
+    }
     R.st_data();
     R.st_data();
     R.st_data();
@@ -1061,13 +1092,21 @@ void cull_chain_host(st_ctx *c, st_cull_params *cp, CullRun &R)
     R.smooth();
     if (cp->islandThresh > 0)
         R.islands();
-    R.get(cp->offR, R.D.offR, R.n);
-    R.get(cp->offA, R.D.offA, R.n);
-    R.get(cp->type, R.D.type, R.n);
-    R.get(cp->sigmaR, R.D.sigmaR, R.n);
-    R.get(cp->sigmaA, R.D.sigmaA, R.n);
-    R.get(cp->offRS, R.D.offRS, R.n);
-    R.get(cp->offAS, R.D.offAS, R.n);
+    if (staged) {
+        ST_HIP(hipMemcpyAsync(stg, dev, all, hipMemcpyDeviceToHost, c->stream));
+        ST_HIP(hipStreamSynchronize(c->stream));
+        parallel_copy({{cp->offR, at(D.offR), f4}, {cp->offA, at(D.offA), f4}, {cp->type, at(D.type), (size_t)R.n},
+                       {cp->sigmaR, at(D.sigmaR), f4}, {cp->sigmaA, at(D.sigmaA), f4}, {cp->offRS, at(D.offRS), f4},
+                       {cp->offAS, at(D.offAS), f4}});
+        return;
+    }
+    R.get(cp->offR, D.offR, R.n);
+    R.get(cp->offA, D.offA, R.n);
+    R.get(cp->type, D.type, R.n);
+    R.get(cp->sigmaR, D.sigmaR, R.n);
+    R.get(cp->sigmaA, D.sigmaA, R.n);
+    R.get(cp->offRS, D.offRS, R.n);
+    R.get(cp->offAS, D.offAS, R.n);
     ST_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -1117,7 +1156,7 @@ extern "C" int st_cull_run(st_ctx *c, st_cull_params *cp)
     return st_guard(c, [&]() {
         CullRun R(c, cp);
         ST_REQUIRE(cull_arrays(cp), ST_ERR_ARG, "cull arrays");
-        cull_chain_host(c, cp, R);
+        cull_chain_host(c, cp, R, true);
     });
 }
 
@@ -1135,7 +1174,7 @@ extern "C" int st_cull_run_noalloc(st_ctx *c, st_cull_params *cp)
         void *base = (c->device >= 0 && c->device < kMaxDevices) ? gScratch[c->device] : nullptr;
         ST_REQUIRE(base, ST_ERR_HIP, "cull scratch array not set up on this device");
         CullRun R(c, cp, base, kNoAllocBytes);
-        cull_chain_host(c, cp, R);
+        cull_chain_host(c, cp, R, false);  // allocates nothing, pinned host memory included
     });
 }
 
