@@ -1,0 +1,118 @@
+// Register transforms of length N = 128, 192, 256, 384, 512, 768 on
+// LANES = N / V adjacent lanes of one wave, V = 8 values per lane (powers of
+// two) or 24 (three times a power of two): lane j holds x[j + LANES i],
+// i = 0 .. V - 1, on entry and on return.  Stages, twiddle values and product
+// contractions are those of stfft::Engine's plan for N (as fft8, whose exchange
+// through a private LDS region of N + N / 8 elements it shares), so the
+// results are bit-identical to its LDS passes.
+#pragma once
+
+#include "st_fft8.h"
+
+namespace fftn {
+
+// exp(-2 pi i e / 512) and exp(-2 pi i e / 768)
+extern __constant__ float2 c_tw512[512], c_tw768[768];
+
+template <int N>
+struct Plan {
+    static_assert(N == 128 || N == 192 || N == 256 || N == 384 || N == 512 || N == 768, "transform length");
+    static constexpr int V = N % 3 ? 8 : 24, LANES = N / V, REGION = N + N / 8;
+};
+
+inline bool covered(int n) { return n == 128 || n == 192 || n == 256 || n == 384; }
+
+template <int N>
+__device__ inline float2 twiddle(int e)  // exp(-2 pi i e / N)
+{
+    if constexpr (N % 3 == 0)
+        return c_tw768[e * (768 / N)];
+    else
+        return c_tw512[e * (512 / N)];
+}
+
+template <int SIGN>
+__device__ inline void dft3(float2 &a, float2 &b, float2 &d)
+{
+#pragma clang fp contract(off)
+    const float c = -0.5f, s = 0.86602540378443864676f * SIGN;
+    const float2 t1 = cadd(b, d), t2 = csub(b, d);
+    const float2 m = make_float2(fmaf(c, t1.x, a.x), fmaf(c, t1.y, a.y));
+    a = cadd(a, t1);
+    b = make_float2(fmaf(-s, t2.y, m.x), fmaf(s, t2.x, m.y));
+    d = make_float2(fmaf(s, t2.y, m.x), fmaf(-s, t2.x, m.y));
+}
+
+// One stage: butterflies jj = j + LANES u, u < V / R, on elements u + (V / R) r.
+template <int N, int R, int NS, int SIGN>
+__device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex)
+{
+    constexpr int V = Plan<N>::V, LANES = Plan<N>::LANES, NB = V / R;
+    static_assert(NB * R == V, "radix divides the lane's values");
+#pragma unroll
+    for (int u = 0; u < NB; u++) {
+        const int k = (j + LANES * u) % NS;
+        if constexpr (NS > 1) {
+#pragma unroll
+            for (int r = 1; r < R; r++)
+                v[u + NB * r] = fft8::mul_tw<SIGN>(v[u + NB * r], twiddle<N>(k * r * (N / (NS * R))));
+        }
+        if constexpr (R == 8) {
+            float2 w[8];
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+                w[r] = v[u + NB * r];
+            fft8::dft8<SIGN>(w);
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+                v[u + NB * r] = w[r];
+        } else if constexpr (R == 4) {
+            stfft::dft4(v[u], v[u + NB], v[u + 2 * NB], v[u + 3 * NB], SIGN);
+        } else {
+            dft3<SIGN>(v[u], v[u + NB], v[u + 2 * NB]);
+        }
+    }
+    if constexpr (NS * R < N) {
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int jj = j + LANES * u, at = (jj / NS) * NS * R + jj % NS;
+#pragma unroll
+            for (int q = 0; q < R; q++)
+                ex[fft8::pad(at + q * NS)] = v[u + NB * q];
+        }
+        fft8::wave_sync();
+#pragma unroll
+        for (int i = 0; i < V; i++)
+            v[i] = ex[fft8::pad(j + LANES * i)];
+        fft8::wave_sync();
+    }
+}
+
+template <int N, int SIGN>
+__device__ inline void fft(float2 (&v)[Plan<N>::V], int j, float2 *ex)
+{
+    stage<N, 8, 1, SIGN>(v, j, ex);
+    if constexpr (N == 128) {
+        stage<N, 4, 8, SIGN>(v, j, ex);
+        stage<N, 4, 32, SIGN>(v, j, ex);
+    } else if constexpr (N == 192) {
+        stage<N, 8, 8, SIGN>(v, j, ex);
+        stage<N, 3, 64, SIGN>(v, j, ex);
+    } else if constexpr (N == 256) {
+        stage<N, 8, 8, SIGN>(v, j, ex);
+        stage<N, 4, 64, SIGN>(v, j, ex);
+    } else if constexpr (N == 384) {
+        stage<N, 4, 8, SIGN>(v, j, ex);
+        stage<N, 4, 32, SIGN>(v, j, ex);
+        stage<N, 3, 128, SIGN>(v, j, ex);
+    } else if constexpr (N == 512) {
+        stage<N, 8, 8, SIGN>(v, j, ex);
+        stage<N, 8, 64, SIGN>(v, j, ex);
+    } else {
+        stage<N, 8, 8, SIGN>(v, j, ex);
+        stage<N, 4, 64, SIGN>(v, j, ex);
+        stage<N, 3, 256, SIGN>(v, j, ex);
+    }
+}
+
+}  // namespace fftn

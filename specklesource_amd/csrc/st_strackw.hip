@@ -21,13 +21,19 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "st_ctx.h"
 #include "st_fftlds.h"
+#include "st_fftn.h"
 #include "st_track_common.h"
 
 using namespace sttrack;
+
+namespace fftn {
+__constant__ float2 c_tw512[512], c_tw768[768];
+}
 
 namespace {
 
@@ -318,6 +324,8 @@ __global__ void __launch_bounds__(NT) k_w_colinterp(WPar p, WBatch Bt, int B, in
     }
 }
 
+#include "st_strackw_fixed.h"
+
 #pragma clang fp contract(off)
 // detectPatch (corrTrackFast.c:765-839) of the search (image 1, whole
 // array, boxcar clamped to the array) and the chip (image 2, inner region,
@@ -405,7 +413,9 @@ size_t detect_lds_bytes(const WPar &p)
 
 // Chip mean and variance (computeMeanSigma, corrTrackFast.c:418-431):
 // sigma = sum(d^2)/(N-1) - mean^2.
-__global__ void __launch_bounds__(NT) k_w_chipstats(WPar p, WBatch Bt)
+// FIXED: on k_wf_detect's chip image in place of Z.
+template <bool FIXED>
+__global__ void __launch_bounds__(NT) k_w_chipstats(WPar p, WBatch Bt, WfBatch F)
 {
     __shared__ double sh[NT / 64];
     const int b = blockIdx.x;
@@ -414,7 +424,7 @@ __global__ void __launch_bounds__(NT) k_w_chipstats(WPar p, WBatch Bt)
     double s1 = 0.0, s2 = 0.0;
     for (int e = threadIdx.x; e < n; e += NT) {
         const int i = e / p.wR2, j = e - (e / p.wR2) * p.wR2;
-        const float d = Zb[(size_t)(p.epA * WOS + i) * p.W_R + p.epR * WOS + j].y;
+        const float d = FIXED ? F.Cf[(size_t)b * n + e] : Zb[(size_t)(p.epA * WOS + i) * p.W_R + p.epR * WOS + j].y;
         s1 += d;
         s2 += d * d;
     }
@@ -485,9 +495,10 @@ __device__ inline void top2_merge(double &best, double &second, int &rank, doubl
 // window sums come from an exclusive prefix over the columns (in
 // LDS, one slice per row of the round).  NCC in FP64; best and runner-up
 // within the searched lags (rank = row-major lag index, the reference's
-// first-maximum rule) per row.
-template <int PER>
-__global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, int nRun, int nStep)
+// first-maximum rule) per row.  FIXED: search image and correlation from Sf
+// and Gf in place of Z and U.
+template <int PER, bool FIXED>
+__global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, WfBatch F, int nRun, int nStep)
 {
     extern __shared__ double lds[];
     __shared__ double sh[4][2 * kNccStep];
@@ -496,8 +507,11 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, int nRun, int 
     const int b = blockIdx.y, run = blockIdx.x;
     const int i0 = run * kNccRows, i1 = imin(i0 + kNccRows, p.nLagA);
     const int slice = 2 * (p.W_R + 1);
-    const float2 *Zb = Bt.Z + (size_t)b * p.W_A * p.W_R;
     const int NN = p.W_A * p.W_R;
+    auto search = [&](int row, int c) {
+        const size_t e = (size_t)b * NN + (size_t)row * p.W_R + c;
+        return FIXED ? F.Sf[e] : Bt.Z[e].x;
+    };
     const float2 *Xb = Bt.U + (size_t)(b >> 1) * NN;
     const bool odd = b & 1;
     const int nTile = (p.W_A + kTile - 1) / kTile;
@@ -515,7 +529,7 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, int nRun, int 
                 v2[k] += cs[(size_t)j * 2 * p.W_R + p.W_R + c];
             }
             for (int l = jB * kTile; l < i0 + p.wA2; l++) {
-                const float d = Zb[(size_t)l * p.W_R + c].x;
+                const float d = search(l, c);
                 v1[k] += d;
                 v2[k] += d * d;
             }
@@ -533,12 +547,11 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, int nRun, int 
             const int i = ib + r;
             if (r < nr) {
                 if (i > i0) {
-                    const float2 *top = Zb + (size_t)(i - 1) * p.W_R, *bot = Zb + (size_t)(i - 1 + p.wA2) * p.W_R;
 #pragma unroll
                     for (int k = 0; k < PER; k++) {
                         const int c = threadIdx.x + 256 * k;
                         if (c < p.W_R) {
-                            const float e = top[c].x, d = bot[c].x;
+                            const float e = search(i - 1, c), d = search(i - 1 + p.wA2, c);
                             v1[k] -= e;
                             v2[k] -= e * e;
                             v1[k] += d;
@@ -630,8 +643,13 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, int nRun, int 
                     const double m = (P1[s + p.wR2] - P1[s]) / N;
                     const double sig = (P2[s + p.wR2] - P2[s]) / (N - 1.) - m * m;
                     const int c = s - WOS * p.epR;
-                    const float2 xv = X[(c + p.W_R) % p.W_R];
-                    const float v = odd ? xv.y : xv.x;
+                    float v;
+                    if constexpr (FIXED) {
+                        v = F.Gf[((size_t)b * p.nLagA + i) * p.nLagR + s];
+                    } else {
+                        const float2 xv = X[(c + p.W_R) % p.W_R];
+                        v = odd ? xv.y : xv.x;
+                    }
                     const float mag = sqrtf(v * v);  // = (float)sqrt((double)(v * v)), bit for bit
                     double cr = (double)mag * p.scaleW;
                     cr = cr - meanR * m;
@@ -886,6 +904,15 @@ void init_dirichlet_w(st_ctx *ctx)
         h[k] = (double)s;
     }
     ST_HIP(hipMemcpyToSymbol(HIP_SYMBOL(c_dirw), h, sizeof(h)));
+    auto roots = [](float2 *t, int n) {
+        for (int j = 0; j < n; j++)
+            t[j] = make_float2((float)cos(-2.0 * M_PI * (double)j / n), (float)sin(-2.0 * M_PI * (double)j / n));
+    };
+    float2 tw[768];
+    roots(tw, 512);
+    ST_HIP(hipMemcpyToSymbol(HIP_SYMBOL(fftn::c_tw512), tw, sizeof(float2) * 512));
+    roots(tw, 768);
+    ST_HIP(hipMemcpyToSymbol(HIP_SYMBOL(fftn::c_tw768), tw, sizeof(float2) * 768));
     done[ctx->device] = true;
 }
 
@@ -966,9 +993,15 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
 
     if (nList > 0) {
         const size_t NN = (size_t)p.W_A * p.W_R;
-        // interpolation blocking: R rows per k_w_rowinterp block, C columns
-        // per k_w_colinterp block
-        const int R = std::max(1, std::min(p.wAa, kRowElems / p.W_R));
+        // The fixed-size passes take the sizes they are built for: there they
+        // beat the general ones (750 points of 128^2 windows 2.58 -> 1.84 ms,
+        // 576 of 384^2 18.6 -> 11.8 ms); the general ones stay for all others,
+        // and on request.
+        const char *path = getenv("SPECKLE_AMD_PATH");
+        const bool fixed = wf_covered(p) && !(path && strcmp(path, "staged") == 0);
+        // interpolation blocking of the general passes: R rows per
+        // k_w_rowinterp block, C columns per k_w_colinterp block
+        const int R = fixed ? wf_rows_per_block(p.wRa) : std::max(1, std::min(p.wAa, kRowElems / p.W_R));
         ST_REQUIRE(p.W_R <= kRowElems && p.W_A <= kColElems, ST_ERR_UNSUPPORTED, "window too large for the FFT blocks");
         int lc = 0;
         while ((2 << lc) <= 16 && (2 << lc) * p.W_A <= kColElems)
@@ -976,7 +1009,8 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
         const int C = 1 << lc;
         const int nblk = (p.wAa + R - 1) / R;
         const int nRun = (p.nLagA + kNccRows - 1) / kNccRows;
-        const size_t per = 2 * NN * 8 + 2 * NN * 8 + (size_t)p.nLagA * p.nLagR * 4 +
+        const size_t images = fixed ? NN * 4 + (size_t)p.wA2 * p.wR2 * 4 : 2 * NN * 8;
+        const size_t per = 2 * NN * 8 + images + (size_t)p.nLagA * p.nLagR * 4 +
                            (size_t)p.nLagA * sizeof(RowBest) + 2 * (size_t)(nblk + 1) * 32 +
                            (size_t)((p.W_A + kTile - 1) / kTile) * 2 * p.W_R * 8 + 4096;
         // a batch the device cannot hold is halved until it fits
@@ -999,11 +1033,25 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
         ST_HIP(hipMemcpyAsync(dPos, pos.data(), nList * sizeof(int4), hipMemcpyHostToDevice, st));
         WBatch Bt{};
         Bt.pos = dPos;
-        Bt.U = ar.take<float2>(2 * (size_t)B * NN);
-        float2 *TMP = ar.take<float2>(2 * (size_t)B * NN);
-        Bt.Z = TMP;
-        Bt.Zs = TMP + (size_t)B * NN;  // Z stays intact for the window sums of k_w_ncc
-        Bt.T = TMP;  // [2][B][wAa][W_R] fits: consumed before k_w_detect writes Z
+        float2 *TMP = nullptr;
+        WfBatch F{};
+        if (fixed) {
+            // U, G and Gf follow each other in one buffer, T, Zs and X in the other
+            float2 *A = ar.take<float2>((size_t)B * NN), *T = ar.take<float2>((size_t)B * NN);
+            F.U = (float *)A;
+            F.G = A;
+            F.Gf = (float *)A;
+            Bt.T = Bt.Zs = F.X = T;
+            F.Sf = ar.take<float>((size_t)B * NN);
+            F.Cf = ar.take<float>((size_t)B * p.wA2 * p.wR2);
+            F.pitchX = (p.nLagR + 15) / 16 * 16;
+        } else {
+            Bt.U = ar.take<float2>(2 * (size_t)B * NN);
+            TMP = ar.take<float2>(2 * (size_t)B * NN);
+            Bt.Z = TMP;
+            Bt.Zs = TMP + (size_t)B * NN;  // Z stays intact for the window sums of k_w_ncc
+            Bt.T = TMP;  // [2][B][wAa][W_R] fits: consumed before k_w_detect writes Z
+        }
         Bt.dop = ar.take<double>(2 * (size_t)B * nblk * 4);
         Bt.dopE = ar.take<double>(2 * (size_t)B * 4);
         Bt.chip = ar.take<double>(2 * (size_t)B);
@@ -1022,35 +1070,81 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
             const int nb = std::min(B, nList - off);
             const int np = (nb + 1) / 2;
             Bt.res = dRes + off;
-            ctx->time_begin(kFftSlot);
-            hipLaunchKernelGGL(k_w_rowinterp, dim3(nblk, 2 * nb), dim3(NT), ldsRow, st, p, off, Bt, nb, R, PfR, PiR);
-            hipLaunchKernelGGL(k_w_az, dim3(nb), dim3(64), 0, st, p, Bt, nb, nblk);
-            hipLaunchKernelGGL(k_w_colinterp, dim3((p.W_R + C - 1) / C, 2 * nb), dim3(NT), ldsCol, st, p, Bt, nb, lc,
-                               PfA, PiA);
-            ctx->time_end(kFftSlot);
-            ctx->time_begin(kDet);
-            hipLaunchKernelGGL(k_w_detect, dim3((p.W_R + kTile - 1) / kTile, (p.W_A + kTile - 1) / kTile, nb),
-                               dim3(256), detect_lds_bytes(p), st, p, Bt, nb);
-            ctx->time_end(kDet);
-            ctx->time_begin(kStat);
-            hipLaunchKernelGGL(k_w_chipstats, dim3(nb), dim3(NT), 0, st, p, Bt);
-            ctx->time_end(kStat);
-            ctx->time_begin(kFftSlot);
-            ctx->fft.fft2d_to(Bt.Z, Bt.Zs, nb, p.W_A, p.W_R, -1, st);
-            ctx->time_end(kFftSlot);
-            hipLaunchKernelGGL(k_w_cross, dim3((unsigned)((NN + 255) / 256), np), dim3(256), 0, st, p, Bt, nb);
-            ctx->time_begin(kFftSlot);
-            ctx->fft.fft2d(Bt.U, TMP, np, p.W_A, p.W_R, +1, st);
-            ctx->time_end(kFftSlot);
-            ctx->time_begin(kNcc);
-            {
-                const dim3 g(nRun, nb);
+            const dim3 gDet((p.W_R + kTile - 1) / kTile, (p.W_A + kTile - 1) / kTile, nb), gNcc(nRun, nb);
+            if (fixed) {
+                ctx->time_begin(kFftSlot);
+                wf_size(p.wRa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    hipLaunchKernelGGL(k_wf_rows<decltype(n)::value>, dim3(nblk, 2 * nb), dim3(G::NTHR), G::LDSR, st, p,
+                                       off, Bt, nb);
+                });
+                hipLaunchKernelGGL(k_w_az, dim3(nb), dim3(64), 0, st, p, Bt, nb, nblk);
+                wf_size(p.wAa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    const int2 cc = wf_chip_cols(p);
+                    const int nb0 = p.W_R / G::C, nb1 = (cc.y + G::C - 1) / G::C - cc.x / G::C;
+                    hipLaunchKernelGGL(k_wf_cols<decltype(n)::value>, dim3(nb0 + nb1, nb), dim3(G::NTHC), G::LDSC, st, p,
+                                       Bt, F, nb, nb0);
+                });
+                ctx->time_end(kFftSlot);
+                ctx->time_begin(kDet);
+                hipLaunchKernelGGL(k_wf_detect, gDet, dim3(256), detect_lds_bytes(p), st, p, Bt, F, nb);
+                ctx->time_end(kDet);
+                ctx->time_begin(kStat);
+                hipLaunchKernelGGL(k_w_chipstats<true>, dim3(nb), dim3(NT), 0, st, p, Bt, F);
+                ctx->time_end(kStat);
+                ctx->time_begin(kFftSlot);
+                wf_size(p.wRa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    hipLaunchKernelGGL(k_wf_zrows<decltype(n)::value>, dim3(p.W_A / G::R, nb), dim3(G::NTHR), G::LDSR,
+                                       st, p, Bt, F);
+                });
+                wf_size(p.wAa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    hipLaunchKernelGGL(k_wf_cross<decltype(n)::value>, dim3(p.W_R / 2 / G::C, np), dim3(G::NTHC), G::LDSC,
+                                       st, p, Bt, F, nb);
+                });
+                wf_size(p.wRa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    hipLaunchKernelGGL(k_wf_urows<decltype(n)::value>, dim3(p.W_A / G::R, np), dim3(G::NTHR), G::LDSR,
+                                       st, p, F);
+                });
+                wf_size(p.wAa, [&](auto n) {
+                    using G = WfGeom<decltype(n)::value>;
+                    hipLaunchKernelGGL(k_wf_lags<decltype(n)::value>, dim3((p.nLagR + G::C - 1) / G::C, np),
+                                       dim3(G::NTHC), G::LDSC, st, p, F, nb);
+                });
+                ctx->time_end(kFftSlot);
+                ctx->time_begin(kNcc);
+                hipLaunchKernelGGL((k_w_ncc<4, true>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
+                ctx->time_end(kNcc);
+            } else {
+                ctx->time_begin(kFftSlot);
+                hipLaunchKernelGGL(k_w_rowinterp, dim3(nblk, 2 * nb), dim3(NT), ldsRow, st, p, off, Bt, nb, R, PfR, PiR);
+                hipLaunchKernelGGL(k_w_az, dim3(nb), dim3(64), 0, st, p, Bt, nb, nblk);
+                hipLaunchKernelGGL(k_w_colinterp, dim3((p.W_R + C - 1) / C, 2 * nb), dim3(NT), ldsCol, st, p, Bt, nb, lc,
+                                   PfA, PiA);
+                ctx->time_end(kFftSlot);
+                ctx->time_begin(kDet);
+                hipLaunchKernelGGL(k_w_detect, gDet, dim3(256), detect_lds_bytes(p), st, p, Bt, nb);
+                ctx->time_end(kDet);
+                ctx->time_begin(kStat);
+                hipLaunchKernelGGL(k_w_chipstats<false>, dim3(nb), dim3(NT), 0, st, p, Bt, F);
+                ctx->time_end(kStat);
+                ctx->time_begin(kFftSlot);
+                ctx->fft.fft2d_to(Bt.Z, Bt.Zs, nb, p.W_A, p.W_R, -1, st);
+                ctx->time_end(kFftSlot);
+                hipLaunchKernelGGL(k_w_cross, dim3((unsigned)((NN + 255) / 256), np), dim3(256), 0, st, p, Bt, nb);
+                ctx->time_begin(kFftSlot);
+                ctx->fft.fft2d(Bt.U, TMP, np, p.W_A, p.W_R, +1, st);
+                ctx->time_end(kFftSlot);
+                ctx->time_begin(kNcc);
                 if (p.W_R <= 256 * 4)
-                    hipLaunchKernelGGL(k_w_ncc<4>, g, dim3(256), ldsNcc, st, p, Bt, nRun, nStep);
+                    hipLaunchKernelGGL((k_w_ncc<4, false>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
                 else
-                    hipLaunchKernelGGL(k_w_ncc<8>, g, dim3(256), ldsNcc, st, p, Bt, nRun, nStep);
+                    hipLaunchKernelGGL((k_w_ncc<8, false>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
+                ctx->time_end(kNcc);
             }
-            ctx->time_end(kNcc);
             ctx->time_begin(kRef);
             hipLaunchKernelGGL(k_w_refine, dim3(nb), dim3(256), 0, st, p, Bt);
             ctx->time_end(kRef);

@@ -1,0 +1,488 @@
+// strackw's passes at fixed window sizes (wRa and wAa each one of 128, 192,
+// 256, 384), included by st_strackw.hip inside its anonymous namespace.  The
+// same transforms as the general kernels, in the same order and with the same
+// roundings (fftn), with less between them:
+//   k_wf_rows    range interpolation of both windows; of the chip's only the
+//                columns its detection reads                      -> T
+//   k_wf_cols    azimuth interpolation, |z|^2 scale               -> U (floats)
+//   k_wf_detect  boxcar, square root: search image s, chip image c, column
+//                sums of s and s^2 over 32-row tiles              -> Sf, Cf
+//   k_wf_zrows   forward range transforms of s + i c              -> Zs
+//   k_wf_cross   forward azimuth transforms of columns l and -l of two patches,
+//                their cross spectra G0 + i G1                    -> G
+//   k_wf_urows   range inverse, the lag columns only              -> X
+//   k_wf_lags    azimuth inverse of the lag columns: both patches'
+//                correlations at the lags                         -> Gf
+// followed by k_w_ncc and k_w_refine.
+//
+// Values stay in registers between the stages of a transform and images are
+// stored as floats, of the chip only what is read; the general passes exchange
+// every stage through LDS with a block barrier and move complex images.  576
+// windows of 384^2, general -> here: interpolation 6.6 -> 3.2 ms, detection
+// 2.04 -> 1.87, chip statistics 0.16 -> 0.12, correlation transforms with the
+// cross spectra 7.0 -> 4.0, coarse correlation 2.60 -> 2.43.  Bound: LDS
+// exchanges and VALU issue at two waves per SIMD in the interpolation and the
+// cross spectra, HBM in k_wf_zrows, k_wf_urows and k_wf_lags (3.4 to 4.9 TB/s).
+
+// Geometry for window side N: M = 2 N interpolated samples, C columns (or
+// slots) and R rows per workgroup.
+template <int N>
+struct WfGeom {
+    static constexpr int M = 2 * N, VN = fftn::Plan<N>::V, LN = fftn::Plan<N>::LANES;
+    static constexpr int VM = fftn::Plan<M>::V, LM = fftn::Plan<M>::LANES;
+    // an LDS region: N + N / 8 elements, 8 more than a multiple of 32 so that
+    // stores and loads of 8 columns across 8 regions meet no bank twice
+    static constexpr int PB = (M + M / 8 + 23) / 32 * 32 + 8;
+    static constexpr int R = 256 / LM, NTHR = R * LM;
+    static constexpr int C = 8, NTHC = C * LM;
+    static constexpr size_t LDSR = (size_t)R * PB * sizeof(float2), LDSC = (size_t)C * PB * sizeof(float2);
+    static_assert(LM == 2 * LN && VM == VN, "lane groups");
+};
+
+struct WfBatch {
+    float *U;    // [2][B][W_A][W_R] |z|^2 scale of the search, of the chip
+    float *Sf;   // [B][W_A][W_R] search image
+    float *Cf;   // [B][wA2][wR2] chip image
+    float2 *G;   // [(B + 1) / 2][W_A][W_R] cross spectra of two patches
+    float2 *X;   // [(B + 1) / 2][W_A][pitchX] after the range inverse, by lag
+    float *Gf;   // [B][nLagA][nLagR] correlation at the lags
+    int pitchX;  // nLagR rounded up to 16
+};
+
+// Columns of the chip's interpolated image that k_wf_detect reads: its inner
+// region and the boxcar's reach.
+__host__ __device__ inline int2 wf_chip_cols(const WPar &p)
+{
+    const int h = p.navgA > 1 || p.navgR > 1 ? p.navgR : 0, e0 = p.epR * WOS;
+    return make_int2(imax(0, e0 - h), imin(p.W_R, e0 + p.wR2 + h));
+}
+
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WBatch Bt, int B)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VN, NW = G::NTHR / 64;
+    extern __shared__ float2 ldsf[];
+    __shared__ double sh[NW][4];
+    const int z = blockIdx.y, img = z >= B ? 1 : 0, b = z - img * B, t = threadIdx.x;
+    const int4 q = Bt.pos[off + b];
+    const int rr = img ? q.z : q.x, ra = img ? q.w : q.y;
+    const int i0 = blockIdx.x * G::R;
+    double s[4] = {0, 0, 0, 0};  // sum x, sum x[i + 1] conj(x[i]) (re, im)
+    if (t < G::R * G::LN) {
+        const int j = t % G::LN, i = i0 + t / G::LN;
+        float2 *ex = ldsf + (t / G::LN) * G::PB;
+        float2 v[V];
+        const bool next = i + 1 < p.wAa;
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            v[r] = sample0(p.im, img, ra + i, rr + j + G::LN * r);
+#pragma unroll
+        for (int r = 0; r < V; r++) {
+            s[0] += v[r].x;
+            s[1] += v[r].y;
+        }
+        if (i == 0 || !next) {
+            // this row's sum alone (the lanes of the row hold it)
+            double e0 = s[0], e1 = s[1];
+            for (int o = 1; o < G::LN; o <<= 1) {
+                e0 += __shfl_xor(e0, o);
+                e1 += __shfl_xor(e1, o);
+            }
+            if (j == 0) {
+                double *E = Bt.dopE + 4 * z + (i == 0 ? 0 : 2);
+                E[0] = e0;
+                E[1] = e1;
+            }
+        }
+        if (next)
+#pragma unroll
+            for (int r = 0; r < V; r++) {
+                const float2 x1 = sample0(p.im, img, ra + i + 1, rr + j + G::LN * r), x0 = v[r];
+                s[2] += (double)x1.x * x0.x + (double)x1.y * x0.y;
+                s[3] += (double)x1.y * x0.x - (double)x1.x * x0.y;
+            }
+        fftn::fft<N, -1>(v, j, ex);
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            ex[j + G::LN * r] = v[r];
+    }
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            s[k] += __shfl_xor(s[k], o);
+    if ((t & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            sh[t >> 6][k] = s[k];
+    __syncthreads();
+    if (t < 4) {
+        double a = 0;
+        for (int w = 0; w < NW; w++)
+            a += sh[w][t];
+        Bt.dop[((size_t)z * gridDim.x + blockIdx.x) * 4 + t] = a;
+    }
+    const int j = t % G::LM, i = i0 + t / G::LM;
+    float2 *ex = ldsf + (t / G::LM) * G::PB;
+    float2 v[V];
+#pragma unroll
+    for (int r = 0; r < V; r++) {
+        // bins 0 .. N / 2 - 1 stay, the Nyquist bin and the negative
+        // frequencies move to the top, zeros between
+        const int m = j + G::LM * r;
+        v[r] = r < V / 4 ? ex[m] : r >= V - V / 4 ? ex[m - N] : make_float2(0.f, 0.f);
+    }
+    fft8::wave_sync();
+    fftn::fft<G::M, +1>(v, j, ex);
+    const int2 cols = img ? wf_chip_cols(p) : make_int2(0, p.W_R);
+    float2 *T = Bt.T + ((size_t)z * p.wAa + i) * p.W_R;
+#pragma unroll
+    for (int r = 0; r < V; r++) {
+        const int m = j + G::LM * r;
+        if (m >= cols.x && m < cols.y)
+            T[m] = v[r];
+    }
+}
+
+// Workgroups of a patch: column blocks of the search image, then those of the
+// chip's columns.
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, WfBatch F, int B, int nb0)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VN, C = G::C, M = G::M, LM = G::LM, LN = G::LN;
+    extern __shared__ float2 ldsf[];
+    const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
+    const int L = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;  // neighbouring column blocks on one XCD
+    const int b = L / nbx, blk = L - b * nbx, img = blk >= nb0 ? 1 : 0, z = img * B + b, t = threadIdx.x;
+    const int c0 = img ? (wf_chip_cols(p).x / C + blk - nb0) * C : blk * C;
+    const float2 *T = Bt.T + (size_t)z * p.wAa * p.W_R + c0;
+    {
+        constexpr int K = N / LM;
+        float2 u[K];
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            u[k] = T[(size_t)(t / C + k * LM) * p.W_R + t % C];
+#pragma unroll
+        for (int k = 0; k < K; k++)
+            ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
+    }
+    __syncthreads();
+    if (t < C * LN) {
+        const int j = t % LN;
+        float2 *ex = ldsf + (t / LN) * G::PB;
+        float2 v[V];
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            v[r] = ex[j + LN * r];
+        fft8::wave_sync();
+        fftn::fft<N, -1>(v, j, ex);
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            ex[j + LN * r] = v[r];
+    }
+    __syncthreads();
+    {
+        const int j = t % LM, az = Bt.az[b];
+        float2 *ex = ldsf + (t / LM) * G::PB;
+        float2 v[V];
+#pragma unroll
+        for (int r = 0; r < V; r++) {
+            v[r] = make_float2(0.f, 0.f);
+            if (r < V / 4 || r >= V - V / 4) {
+                int k = j + LM * r + (r < V / 4 ? 0 : N - M) + az;  // in [0, 2 N)
+                k -= k >= N ? N : 0;
+                v[r] = ex[k];
+            }
+        }
+        fft8::wave_sync();
+        fftn::fft<M, +1>(v, j, ex);
+        float *exf = (float *)ex;
+#pragma unroll
+        for (int r = 0; r < V; r++) {
+#pragma clang fp contract(off)
+            exf[j + LM * r] = (v[r].x * v[r].x + v[r].y * v[r].y) * p.scale;
+        }
+    }
+    __syncthreads();
+    float *U = F.U + (size_t)z * p.W_A * p.W_R + c0;
+#pragma unroll
+    for (int k = 0; k < M / LM; k++) {
+        const int n = t / C + k * LM;
+        U[(size_t)n * p.W_R + t % C] = ((const float *)(ldsf + (t % C) * G::PB))[n];
+    }
+}
+
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_zrows(WPar p, WBatch Bt, WfBatch F)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VM, LM = G::LM;
+    extern __shared__ float2 ldsf[];
+    const int b = blockIdx.y, t = threadIdx.x, j = t % LM, y = blockIdx.x * G::R + t / LM;
+    const float *S = F.Sf + ((size_t)b * p.W_A + y) * p.W_R + j;
+    const int yc = y - p.epA * WOS, e0 = p.epR * WOS;
+    const float *Cr = F.Cf + ((size_t)b * p.wA2 + yc) * p.wR2 - e0 + j;
+    const bool in = yc >= 0 && yc < p.wA2;
+    float2 v[V];
+#pragma unroll
+    for (int r = 0; r < V; r++) {
+        const int x = j + LM * r;
+        v[r] = make_float2(S[LM * r], in && x >= e0 && x < e0 + p.wR2 ? Cr[LM * r] : 0.f);
+    }
+    fftn::fft<G::M, -1>(v, j, ldsf + (t / LM) * G::PB);
+    float2 *Z = Bt.Zs + ((size_t)b * p.W_A + y) * p.W_R + j;
+#pragma unroll
+    for (int r = 0; r < V; r++)
+        Z[LM * r] = v[r];
+}
+
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_urows(WPar p, WfBatch F)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VM, M = G::M, LM = G::LM;
+    extern __shared__ float2 ldsf[];
+    const int q = blockIdx.y, t = threadIdx.x, j = t % LM, y = blockIdx.x * G::R + t / LM;
+    const float2 *Gq = F.G + ((size_t)q * p.W_A + y) * p.W_R + j;
+    float2 v[V];
+#pragma unroll
+    for (int r = 0; r < V; r++)
+        v[r] = Gq[LM * r];
+    fftn::fft<M, +1>(v, j, ldsf + (t / LM) * G::PB);
+    const int lagR = WOS * p.epR;
+    float2 *X = F.X + ((size_t)q * p.W_A + y) * F.pitchX;
+#pragma unroll
+    for (int r = 0; r < V; r++) {
+        const int m = j + LM * r, s = m <= lagR ? m + lagR : m - M + lagR;
+        if (s >= 0 && s < p.nLagR)
+            X[s] = v[r];
+    }
+}
+
+// Lag columns past nLagR (the last workgroup's) hold whatever X did there;
+// they stay in their own regions and are not stored.
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_lags(WPar p, WfBatch F, int B)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VM, C = G::C, M = G::M, LM = G::LM;
+    extern __shared__ float2 ldsf[];
+    const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
+    const int L = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;
+    const int q = L / nbx, c0 = (L - q * nbx) * C, t = threadIdx.x, j = t % LM;
+    const float2 *X = F.X + (size_t)q * p.W_A * F.pitchX + c0;
+    float2 *ex = ldsf + (t / LM) * G::PB;
+    {
+        float2 u[M / LM];
+#pragma unroll
+        for (int k = 0; k < M / LM; k++)
+            u[k] = X[(size_t)(t / C + k * LM) * F.pitchX + t % C];
+#pragma unroll
+        for (int k = 0; k < M / LM; k++)
+            ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
+    }
+    __syncthreads();
+    float2 v[V];
+#pragma unroll
+    for (int r = 0; r < V; r++)
+        v[r] = ex[j + LM * r];
+    fft8::wave_sync();
+    fftn::fft<M, +1>(v, j, ex);
+#pragma unroll
+    for (int r = 0; r < V; r++)
+        ex[j + LM * r] = v[r];
+    __syncthreads();
+    const int lagA = WOS * p.epA, s = c0 + t % C;
+    float *g0 = F.Gf + (size_t)(2 * q) * p.nLagA * p.nLagR + s, *g1 = g0 + (size_t)p.nLagA * p.nLagR;
+    const bool in = s < p.nLagR, second = 2 * q + 1 < B;
+#pragma unroll
+    for (int k = 0; k < M / LM; k++) {
+        const int n = t / C + k * LM, i = n <= lagA ? n + lagA : n - M + lagA;  // lag row of output n
+        if (in && i >= 0 && i < p.nLagA) {
+            const float2 x = ldsf[(t % C) * G::PB + n];
+            g0[(size_t)i * p.nLagR] = x.x;
+            if (second)
+                g1[(size_t)i * p.nLagR] = x.y;
+        }
+    }
+}
+
+#pragma clang fp contract(off)
+// detectPatch from the detected images (k_w_detect's boxcar, clamps and sums).
+__global__ void __launch_bounds__(256) k_wf_detect(WPar p, WBatch Bt, WfBatch F, int B)
+{
+    extern __shared__ float w_det_lds[];
+    __shared__ float sv[kTile][kTile + 1];
+    const int b = blockIdx.z;
+    const size_t NN = (size_t)p.W_A * p.W_R;
+    const float *U1 = F.U + b * NN, *U2 = F.U + ((size_t)B + b) * NN;
+    const bool box = p.navgA > 1 || p.navgR > 1;
+    const int hA = box ? p.navgA : 0, hR = box ? p.navgR : 0;
+    const int y0 = blockIdx.y * kTile, x0 = blockIdx.x * kTile;
+    const int TH = kTile + 2 * hA, TW = kTile + 2 * hR;
+    float *d1 = w_det_lds, *d2 = w_det_lds + TH * TW;
+    const int c0 = p.epA * WOS, c1 = c0 + p.wA2;  // chip rows [c0, c1)
+    const int e0 = p.epR * WOS, e1 = e0 + p.wR2;  // chip cols [e0, e1)
+    const bool chipTile = y0 < c1 && y0 + kTile > c0 && x0 < e1 && x0 + kTile > e0;
+    const int kmaxC = p.epR * WOS + p.wA2 + p.navgA - 1;
+    const int lmaxC = p.epR * WOS + p.wR2 + p.navgR - 1;
+    const int2 cols = wf_chip_cols(p);
+    for (int t = threadIdx.x; t < TH * TW; t += blockDim.x) {
+        const int ty = t / TW, tx = t - (t / TW) * TW;
+        const int y = y0 - hA + ty, x = x0 - hR + tx;
+        d1[t] = U1[(size_t)imin(imax(y, 0), p.W_A - 1) * p.W_R + imin(imax(x, 0), p.W_R - 1)];
+        if (chipTile) {
+            const int ky2 = imin(imin(imax(y, 0), kmaxC), p.W_A - 1), kx2 = imin(imin(imax(x, 0), lmaxC), p.W_R - 1);
+            // columns outside the chip's reach feed no chip cell
+            d2[t] = kx2 >= cols.x && kx2 < cols.y ? U2[(size_t)ky2 * p.W_R + kx2] : 0.f;
+        }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kTile * kTile; t += blockDim.x) {
+        const int oy = t / kTile, ox = t - (t / kTile) * kTile;
+        const int y = y0 + oy, x = x0 + ox;
+        sv[oy][ox] = 0.f;
+        if (y >= p.W_A || x >= p.W_R)
+            continue;
+        float v1 = 0.f;
+        for (int m = -hA; m <= hA; m++)
+            for (int n = -hR; n <= hR; n++)
+                v1 += d1[(oy + hA + m) * TW + ox + hR + n];
+        if (chipTile && y >= c0 && y < c1 && x >= e0 && x < e1) {
+            float v2 = 0.f;
+            for (int m = -hA; m <= hA; m++)
+                for (int n = -hR; n <= hR; n++)
+                    v2 += d2[(oy + hA + m) * TW + ox + hR + n];
+            F.Cf[((size_t)b * p.wA2 + y - c0) * p.wR2 + x - e0] = sqrtf(v2);
+        }
+        const float sr = sqrtf(v1);
+        sv[oy][ox] = sr;
+        F.Sf[b * NN + (size_t)y * p.W_R + x] = sr;
+    }
+    __syncthreads();
+    if (threadIdx.x < kTile && x0 + (int)threadIdx.x < p.W_R) {
+        double a1 = 0.0, a2 = 0.0;
+        for (int oy = 0; oy < kTile; oy++) {
+            const float v = sv[oy][threadIdx.x];
+            a1 += v;
+            a2 += v * v;
+        }
+        double *cs = Bt.csum + ((size_t)b * gridDim.y + blockIdx.y) * 2 * p.W_R + x0 + threadIdx.x;
+        cs[0] = a1;
+        cs[p.W_R] = a2;
+    }
+}
+// S conj(C) at a frequency from Z there (a) and at its mirror (c): k_w_cross's
+// expressions.
+__device__ inline float2 wf_cross(float2 a, float2 c)
+{
+    const float2 S = make_float2(0.5f * (a.x + c.x), 0.5f * (a.y - c.y));
+    const float2 Cc = make_float2(0.5f * (a.y + c.y), 0.5f * (c.x - a.x));
+    return cmulconj(S, Cc);
+}
+
+// Slot c of a workgroup: column l = c0 + c and its mirror W_R - l (W_R / 2 for
+// l = 0, both their own mirrors) of patches 2 q and 2 q + 1, one lane group.
+// The slot's LDS region holds one column at a time: loads and stores in whole
+// segments of C columns pass through it, and so do the mirrored reads.
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch Bt, WfBatch F, int B)
+{
+    using G = WfGeom<N>;
+    constexpr int V = G::VM, C = G::C, M = G::M, LM = G::LM;
+    extern __shared__ float2 ldsf[];
+    const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
+    const int Lb = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;
+    const int q = Lb / nbx, c0 = (Lb - q * nbx) * C, t = threadIdx.x, W = p.W_R, H = W / 2;
+    const int j = t % LM, slot = t / LM;
+    float2 *ex = ldsf + slot * G::PB;
+    const bool self = c0 + slot == 0;
+    // column of load / store lane t % C on side s (0: l, 1: mirror)
+    auto col = [&](int s) {
+        const int l = c0 + t % C;
+        return s == 0 ? l : l == 0 ? H : W - l;
+    };
+    auto load = [&](const float2 *Z, int s, float2(&v)[V]) {
+        float2 u[M / LM];
+        const int c = col(s);
+#pragma unroll
+        for (int k = 0; k < M / LM; k++)
+            u[k] = Z[(size_t)(t / C + k * LM) * W + c];
+        __syncthreads();  // the region's last readers are done
+#pragma unroll
+        for (int k = 0; k < M / LM; k++)
+            ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            v[r] = ex[j + LM * r];
+        fft8::wave_sync();
+    };
+    float2 g[2][V];  // G0 + i G1 of column l, of its mirror
+    auto patch = [&](auto h) {
+        const float2 *Z = Bt.Zs + (size_t)(2 * q + h) * p.W_A * W;
+        float2 x[V], y[V];
+        load(Z, 0, x);
+        fftn::fft<M, -1>(x, j, ex);
+        load(Z, 1, y);
+        fftn::fft<M, -1>(y, j, ex);
+        // side s: the region takes the column at -l (columns 0 and W_R / 2 are their own)
+        auto side = [&](auto s) {
+            float2(&m)[V] = s == 0 ? x : y;
+#pragma unroll
+            for (int r = 0; r < V; r++)
+                ex[j + LM * r] = self == (s == 0) ? x[r] : y[r];
+            fft8::wave_sync();
+#pragma unroll
+            for (int r = 0; r < V; r++) {
+                const float2 d = wf_cross(m[r], ex[r == 0 && j == 0 ? 0 : M - j - LM * r]);
+                g[s][r] = h == 0 ? d : make_float2(g[s][r].x - d.y, g[s][r].y + d.x);
+            }
+            fft8::wave_sync();
+        };
+        side(std::integral_constant<int, 0>());
+        side(std::integral_constant<int, 1>());
+    };
+    patch(std::integral_constant<int, 0>());
+    if (2 * q + 1 < B)  // the same for the whole workgroup
+        patch(std::integral_constant<int, 1>());
+    float2 *Gq = F.G + (size_t)q * p.W_A * W;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+#pragma unroll
+        for (int r = 0; r < V; r++)
+            ex[j + LM * r] = g[s][r];
+        __syncthreads();
+        const int c = col(s);
+#pragma unroll
+        for (int k = 0; k < M / LM; k++) {
+            const int n = t / C + k * LM;
+            Gq[(size_t)n * W + c] = ldsf[(t % C) * G::PB + n];
+        }
+        __syncthreads();
+    }
+}
+
+#pragma clang fp contract(on)
+
+inline bool wf_covered(const WPar &p) { return fftn::covered(p.wRa) && fftn::covered(p.wAa); }
+
+template <class F>
+void wf_size(int n, F f)
+{
+    switch (n) {
+    case 128: f(std::integral_constant<int, 128>()); break;
+    case 192: f(std::integral_constant<int, 192>()); break;
+    case 256: f(std::integral_constant<int, 256>()); break;
+    default: f(std::integral_constant<int, 384>()); break;
+    }
+}
+
+// Rows per workgroup of k_wf_rows (its Doppler partials).
+inline int wf_rows_per_block(int wRa)
+{
+    int r = 1;
+    wf_size(wRa, [&](auto n) { r = WfGeom<decltype(n)::value>::R; });
+    return r;
+}
