@@ -84,7 +84,7 @@ struct WBatch {
     double *chip;     // [B][2]: chip mean, variance
     double *csum;     // [B][ceil(W_A/32)][2][W_R]: column sums of s, s^2 over 32-row tiles
     float *cr;        // [B][nLagA][nLagR]: NCC surface
-    RowBest *rows;    // [B][nLagA]
+    RowBest *rows;    // [B][runs of kNccRows lag rows]
     int *az;          // [B]
     WRes *res;        // [B]
 };
@@ -470,7 +470,6 @@ __global__ void k_w_cross(WPar p, WBatch Bt, int B)
 }
 
 constexpr int kNccRows = 32;  // lag rows per k_w_ncc block (a multiple of the 32-row tiles)
-constexpr int kNccStep = 4;   // lag rows per round of block barriers
 static_assert(kNccRows % kTile == 0, "NCC runs start on tile rows");
 
 // Top-2 merge with the first-rank tie-break.
@@ -486,41 +485,103 @@ __device__ inline void top2_merge(double &best, double &second, int &rank, doubl
     }
 }
 
+// Inclusive sums over the wave's lanes of n doubles, without the LDS pipe: data
+// parallel primitives move the two halves of each (row shifts by 1, 2, 4, 8,
+// then the rows' and the halves' last lanes broadcast).
+template <int CTRL, int ROWS>
+__device__ inline double dpp_move(double x)
+{
+    const int2 v = __builtin_bit_cast(int2, x);
+    return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, v.x, CTRL, ROWS, 0xf, true),
+                                                __builtin_amdgcn_update_dpp(0, v.y, CTRL, ROWS, 0xf, true)));
+}
+template <int n>
+__device__ inline void wave_scan(double (&x)[n])
+{
+    auto step = [&](auto ctrl, auto rows) {
+#pragma unroll
+        for (int q = 0; q < n; q++)
+            x[q] += dpp_move<ctrl, rows>(x[q]);
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>(), integral_constant<int, 0xf>());
+    step(integral_constant<int, 0x112>(), integral_constant<int, 0xf>());
+    step(integral_constant<int, 0x114>(), integral_constant<int, 0xf>());
+    step(integral_constant<int, 0x118>(), integral_constant<int, 0xf>());
+    step(integral_constant<int, 0x142>(), integral_constant<int, 0xa>());
+    step(integral_constant<int, 0x143>(), integral_constant<int, 0xc>());
+}
+
+// x / n, correctly rounded, from rn = 1 / n rounded (Markstein: the residual of
+// the rounded product is exact).
+__device__ inline double div_by(double x, double n, double rn)
+{
+    const double q = x * rn;
+    return fma(fma(-q, n, x), rn, q);
+}
+
+// x / sqrt(a).  Both from one reciprocal square root: coupled Newton steps
+// (Goldschmidt) give the root g and h = 1 / (2 g), a residual step rounds g,
+// another the quotient.  Zeros, negatives, subnormals, infinities and NaN take
+// the library's forms.
+__device__ inline double div_sqrt(double x, double a)
+{
+    if (!(a > 1e-280 && a < 1e280))
+        return x / sqrt(a);
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y, h = 0.5 * y;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const double e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+    }
+    g = fma(fma(-g, g, a), h, g);
+    return div_by(x, g, h + h);
+}
+
 // computeMeanSigma (corrTrackFast.c:407-477, search part) and getPeakCorr
-// (:862-899) for a run of kNccRows lag rows of one patch, nStep <= kNccStep
-// rows per round of block barriers.  Thread t owns columns t + 256 k,
-// k < PER.  The vertical window sums of s and s^2 (FP64, wA2 rows) start
-// from the 32-row tile column sums of k_w_detect (plus the rows of a last
-// partial tile) and slide down one row at a time; each row's horizontal
-// window sums come from an exclusive prefix over the columns (in
-// LDS, one slice per row of the round).  NCC in FP64; best and runner-up
-// within the searched lags (rank = row-major lag index, the reference's
-// first-maximum rule) per row.  FIXED: search image and correlation from Sf
-// and Gf in place of Z and U.
-template <int PER, bool FIXED>
-__global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, WfBatch F, int nRun, int nStep)
+// (:862-899) for a run of kNccRows lag rows of one patch, STEP rows per round.
+// Thread t owns columns PER t .. PER t + PER - 1.  The vertical window sums of
+// s and s^2 (FP64, wA2 rows) start from the 32-row tile column sums of the
+// detection (plus the rows of a last partial tile) and slide down one row at a
+// time in registers; each row's horizontal window sums come from an exclusive
+// prefix over the columns: the thread's own sums, a scan over the wave, the
+// totals of the lower waves.  NCC in FP64, the round's lags dealt out in
+// row-major order over all threads; each thread keeps the best and the
+// runner-up of its searched lags for the whole run (rank = row-major lag index,
+// the reference's first-maximum rule).  FIXED: search image and correlation
+// from Sf and Gf in place of Z and U.
+//
+// Bound: FP64 issue and the latency between the two barriers of a round.  The
+// next rows' samples are loaded before the lags are computed, divisions by
+// constants and by the root take three and some twenty operations.  576 patches
+// of 513^2 lags (768 columns): 1.30 ms; 2.43 with two LDS passes per prefix,
+// shuffles through LDS for the scans and for every row's two best, and four
+// barriers per round.
+template <int PER, int STEP, bool FIXED>
+__global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, WfBatch F, int nRun)
 {
     extern __shared__ double lds[];
-    __shared__ double sh[4][2 * kNccStep];
-    __shared__ RowBest rb[4][kNccStep];
+    __shared__ double sh[4][2 * STEP];
+    __shared__ RowBest rb[4];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int b = blockIdx.y, run = blockIdx.x;
     const int i0 = run * kNccRows, i1 = imin(i0 + kNccRows, p.nLagA);
-    const int slice = 2 * (p.W_R + 1);
+    const int half = p.W_R + 1, slice = 2 * half;
     const int NN = p.W_A * p.W_R;
+    const int cb = threadIdx.x * PER;
     auto search = [&](int row, int c) {
         const size_t e = (size_t)b * NN + (size_t)row * p.W_R + c;
         return FIXED ? F.Sf[e] : Bt.Z[e].x;
     };
-    const float2 *Xb = Bt.U + (size_t)(b >> 1) * NN;
-    const bool odd = b & 1;
     const int nTile = (p.W_A + kTile - 1) / kTile;
     const double *cs = Bt.csum + (size_t)b * nTile * 2 * p.W_R;
     const int jA = i0 / kTile, jB = (i0 + p.wA2) / kTile;
     double v1[PER], v2[PER];
 #pragma unroll
     for (int k = 0; k < PER; k++) {
-        const int c = threadIdx.x + 256 * k;
+        const int c = cb + k;
         v1[k] = 0.0;
         v2[k] = 0.0;
         if (c < p.W_R) {
@@ -535,167 +596,158 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, WfBatch F, int
             }
         }
     }
-    const int per = (p.W_R + 255) / 256;
-    const int cb = threadIdx.x * per, ce = imin(cb + per, p.W_R);
-    const double N = (double)p.wR2 * p.wA2;
+    const double N = (double)p.wR2 * p.wA2, rN = 1.0 / N, rN1 = 1.0 / (N - 1.);
     const double meanR = Bt.chip[2 * b], sigmaR = Bt.chip[2 * b + 1];
-    for (int ib = i0; ib < i1; ib += nStep) {
-        const int nr = imin(nStep, i1 - ib);
-        // slide the window sums to each row of the round and park them
+    const int sA = WOS * (p.epA - WNFAST / 4), sR = WOS * (p.epR - WNFAST / 4);  // searched lags
+    double best = -1e30, second = -1e30;
+    int rank = 0x7fffffff;
+    float top[STEP][PER], bot[STEP][PER];  // the rows that leave and enter at the round's rows
+    auto fetch = [&](int ib) {
 #pragma unroll
-        for (int r = 0; r < kNccStep; r++) {
-            const int i = ib + r;
-            if (r < nr) {
-                if (i > i0) {
+        for (int r = 0; r < STEP; r++)
 #pragma unroll
-                    for (int k = 0; k < PER; k++) {
-                        const int c = threadIdx.x + 256 * k;
-                        if (c < p.W_R) {
-                            const float e = search(i - 1, c), d = search(i - 1 + p.wA2, c);
-                            v1[k] -= e;
-                            v2[k] -= e * e;
-                            v1[k] += d;
-                            v2[k] += d * d;
-                        }
-                    }
-                }
-                double *P1 = lds + r * slice, *P2 = P1 + (p.W_R + 1);
-#pragma unroll
-                for (int k = 0; k < PER; k++) {
-                    const int c = threadIdx.x + 256 * k;
-                    if (c < p.W_R) {
-                        P1[c] = v1[k];
-                        P2[c] = v2[k];
-                    }
-                }
+            for (int k = 0; k < PER; k++) {
+                const int i = ib + r;
+                const bool in = i > i0 && i < i1 && cb + k < p.W_R;
+                top[r][k] = in ? search(i - 1, cb + k) : 0.f;
+                bot[r][k] = in ? search(i - 1 + p.wA2, cb + k) : 0.f;
             }
-        }
-        __syncthreads();
-        // exclusive prefixes over the columns: P[c] = sum_{t < c} V[t]
-        double a[2 * kNccStep], x[2 * kNccStep];
+    };
+    fetch(i0);
+    for (int ib = i0; ib < i1; ib += STEP) {
+        const int nr = imin(STEP, i1 - ib);
+        // window sums of the round's rows; exclusive prefixes over the columns
+        double w1[STEP][PER], w2[STEP][PER], a[2 * STEP], x[2 * STEP];
 #pragma unroll
-        for (int r = 0; r < kNccStep; r++) {
-            const double *P1 = lds + r * slice, *P2 = P1 + (p.W_R + 1);
+        for (int r = 0; r < STEP; r++) {
             a[2 * r] = 0.0;
             a[2 * r + 1] = 0.0;
-            if (r < nr)
-                for (int c = cb; c < ce; c++) {
-                    a[2 * r] += P1[c];
-                    a[2 * r + 1] += P2[c];
-                }
+#pragma unroll
+            for (int k = 0; k < PER; k++) {
+                const float e = top[r][k], d = bot[r][k];
+                v1[k] -= e;
+                v2[k] -= e * e;
+                v1[k] += d;
+                v2[k] += d * d;
+                w1[r][k] = v1[k];
+                w2[r][k] = v2[k];
+                a[2 * r] += v1[k];
+                a[2 * r + 1] += v2[k];
+            }
             x[2 * r] = a[2 * r];
             x[2 * r + 1] = a[2 * r + 1];
         }
-        for (int o = 1; o < 64; o <<= 1) {
-#pragma unroll
-            for (int q = 0; q < 2 * kNccStep; q++) {
-                const double u = __shfl_up(x[q], o);
-                if (lane >= o)
-                    x[q] += u;
-            }
-        }
+        wave_scan(x);
         if (lane == 63)
 #pragma unroll
-            for (int q = 0; q < 2 * kNccStep; q++)
+            for (int q = 0; q < 2 * STEP; q++)
                 sh[wid][q] = x[q];
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 2 * kNccStep; q++) {
+        for (int q = 0; q < 2 * STEP; q++) {
             double pre = 0.0;
             for (int w = 0; w < wid; w++)
                 pre += sh[w][q];
-            x[q] += pre - a[q];  // exclusive prefix at the start of the chunk
+            x[q] += pre - a[q];
         }
 #pragma unroll
-        for (int r = 0; r < kNccStep; r++) {
-            if (r < nr) {
-                double *P1 = lds + r * slice, *P2 = P1 + (p.W_R + 1);
-                double r1 = x[2 * r], r2 = x[2 * r + 1];
-                for (int c = cb; c < ce; c++) {
-                    const double u1 = P1[c], u2 = P2[c];
+        for (int r = 0; r < STEP; r++) {
+            double *P1 = lds + r * slice, *P2 = P1 + half;
+            double r1 = x[2 * r], r2 = x[2 * r + 1];
+#pragma unroll
+            for (int k = 0; k < PER; k++) {
+                const int c = cb + k;
+                if (c < p.W_R) {
                     P1[c] = r1;
                     P2[c] = r2;
-                    r1 += u1;
-                    r2 += u2;
                 }
-                if (threadIdx.x == 255) {
+                r1 += w1[r][k];
+                r2 += w2[r][k];
+                if (c == p.W_R - 1) {
                     P1[p.W_R] = r1;
                     P2[p.W_R] = r2;
                 }
             }
         }
         __syncthreads();
-        double best[kNccStep], second[kNccStep];
-        int rank[kNccStep];
-#pragma unroll
-        for (int r = 0; r < kNccStep; r++) {
-            best[r] = -1e30;
-            second[r] = -1e30;
-            rank[r] = 0x7fffffff;
-            const int i = ib + r;
-            if (r < nr) {
-                const double *P1 = lds + r * slice, *P2 = P1 + (p.W_R + 1);
-                const int l = i - WOS * p.epA;
-                const bool rowIn = l >= -WOS * (p.epA - WNFAST / 4) && l <= WOS * (p.epA - WNFAST / 4);
-                const float2 *X = Xb + (size_t)((l + p.W_A) % p.W_A) * p.W_R;
-                float *crRow = Bt.cr + ((size_t)b * p.nLagA + i) * p.nLagR;
-                for (int s = threadIdx.x; s < p.nLagR; s += 256) {
-                    const double m = (P1[s + p.wR2] - P1[s]) / N;
-                    const double sig = (P2[s + p.wR2] - P2[s]) / (N - 1.) - m * m;
-                    const int c = s - WOS * p.epR;
-                    float v;
-                    if constexpr (FIXED) {
-                        v = F.Gf[((size_t)b * p.nLagA + i) * p.nLagR + s];
-                    } else {
-                        const float2 xv = X[(c + p.W_R) % p.W_R];
-                        v = odd ? xv.y : xv.x;
-                    }
-                    const float mag = sqrtf(v * v);  // = (float)sqrt((double)(v * v)), bit for bit
-                    double cr = (double)mag * p.scaleW;
-                    cr = cr - meanR * m;
-                    cr = cr / sqrt(sigmaR * sig);
-                    crRow[s] = (float)cr;
-                    if (rowIn && c >= -WOS * (p.epR - WNFAST / 4) && c <= WOS * (p.epR - WNFAST / 4)) {
-                        if (cr > best[r]) {
-                            second[r] = best[r];
-                            best[r] = cr;
-                            rank[r] = i * p.nLagR + s;
-                        } else if (cr > second[r]) {
-                            second[r] = cr;
-                        }
-                    }
+        fetch(ib + STEP);
+        const size_t e0 = ((size_t)b * p.nLagA + ib) * p.nLagR;
+        int s = threadIdx.x, r = 0;
+        for (int e = threadIdx.x; e < nr * p.nLagR; e += 256, s += 256) {
+            while (s >= p.nLagR) {
+                s -= p.nLagR;
+                r++;
+            }
+            const double *P1 = lds + r * slice + s, *P2 = P1 + half;
+            const int l = ib + r - WOS * p.epA, c = s - WOS * p.epR;
+            float v;
+            if constexpr (FIXED) {
+                v = F.Gf[e0 + e];
+            } else {
+                const float2 xv = Bt.U[(size_t)(b >> 1) * NN + (size_t)(l < 0 ? l + p.W_A : l) * p.W_R +
+                                       (c < 0 ? c + p.W_R : c)];
+                v = b & 1 ? xv.y : xv.x;
+            }
+            const double m = div_by(P1[p.wR2] - P1[0], N, rN);
+            const double sig = div_by(P2[p.wR2] - P2[0], N - 1., rN1) - m * m;
+            const float mag = sqrtf(v * v);  // = (float)sqrt((double)(v * v)), bit for bit
+            double cr = (double)mag * p.scaleW;
+            cr = cr - meanR * m;
+            cr = div_sqrt(cr, sigmaR * sig);
+            Bt.cr[e0 + e] = (float)cr;
+            if (l >= -sA && l <= sA && c >= -sR && c <= sR) {
+                if (cr > best) {
+                    second = best;
+                    best = cr;
+                    rank = ib * p.nLagR + e;
+                } else if (cr > second) {
+                    second = cr;
                 }
             }
         }
-        // top-2 with first-rank tie-break across the block
-        for (int o = 32; o > 0; o >>= 1) {
-#pragma unroll
-            for (int r = 0; r < kNccStep; r++) {
-                const double ob = __shfl_xor(best[r], o), os = __shfl_xor(second[r], o);
-                const int orank = __shfl_xor(rank[r], o);
-                top2_merge(best[r], second[r], rank[r], ob, os, orank);
-            }
-        }
-        if (lane == 0)
-#pragma unroll
-            for (int r = 0; r < kNccStep; r++)
-                rb[wid][r] = RowBest{best[r], second[r], rank[r], 0};
-        __syncthreads();
-        if (threadIdx.x < nr) {
-            const int r = threadIdx.x;
-            RowBest q = rb[0][r];
-            for (int w = 1; w < 4; w++)
-                top2_merge(q.v, q.second, q.rank, rb[w][r].v, rb[w][r].second, rb[w][r].rank);
-            Bt.rows[(size_t)b * p.nLagA + ib + r] = q;
-        }
+    }
+    // top-2 with first-rank tie-break across the block
+    for (int o = 32; o > 0; o >>= 1) {
+        const double ob = __shfl_xor(best, o), os = __shfl_xor(second, o);
+        const int orank = __shfl_xor(rank, o);
+        top2_merge(best, second, rank, ob, os, orank);
+    }
+    if (lane == 0)
+        rb[wid] = RowBest{best, second, rank, 0};
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        RowBest q = rb[0];
+        for (int w = 1; w < 4; w++)
+            top2_merge(q.v, q.second, q.rank, rb[w].v, rb[w].second, rb[w].rank);
+        Bt.rows[(size_t)b * nRun + run] = q;
     }
 }
 
-// Peak over all lag rows, then correlateFast's refinement
+// f(columns per thread, rows per round) of k_w_ncc: the prefixes of a round fit
+// 64 KB of LDS.
+template <class F>
+void ncc_size(int W, F f)
+{
+    using std::integral_constant;
+    if (W <= 256)
+        f(integral_constant<int, 1>(), integral_constant<int, 4>());
+    else if (W <= 512)
+        f(integral_constant<int, 2>(), integral_constant<int, 4>());
+    else if (W <= 768)
+        f(integral_constant<int, 3>(), integral_constant<int, 4>());
+    else if (W <= 1024)
+        f(integral_constant<int, 4>(), integral_constant<int, 3>());
+    else if (W <= 1536)
+        f(integral_constant<int, 6>(), integral_constant<int, 2>());
+    else
+        f(integral_constant<int, 8>(), integral_constant<int, 1>());
+}
+
+// Peak over all runs of lag rows, then correlateFast's refinement
 // (corrTrackFast.c:482-551, 951-990): the 21 x 21 NCC neighbourhood is
 // interpolated by its 16x spectral zero pad, evaluated in FP64 on the
 // searched 64 x 64 window only, Q = A C A^T with A[u][m] = D(136 + u - 16 m).
-__global__ void __launch_bounds__(256) k_w_refine(WPar p, WBatch Bt)
+__global__ void __launch_bounds__(256) k_w_refine(WPar p, WBatch Bt, int nRun)
 {
     __shared__ double dir[kDirN];
     __shared__ float c[kN21 * kN21];
@@ -708,8 +760,8 @@ __global__ void __launch_bounds__(256) k_w_refine(WPar p, WBatch Bt)
         dir[k] = c_dirw[k];
     if (threadIdx.x == 0) {
         RowBest r{-1e30, -1e30, 0x7fffffff, 0};
-        const RowBest *rows = Bt.rows + (size_t)b * p.nLagA;
-        for (int i = 0; i < p.nLagA; i++) {
+        const RowBest *rows = Bt.rows + (size_t)b * nRun;
+        for (int i = 0; i < nRun; i++) {
             const RowBest o = rows[i];
             const bool takeOther = o.v > r.v || (o.v == r.v && o.rank < r.rank);
             const double lo = takeOther ? r.v : o.v;
@@ -1011,7 +1063,7 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
         const int nRun = (p.nLagA + kNccRows - 1) / kNccRows;
         const size_t images = fixed ? NN * 4 + (size_t)p.wA2 * p.wR2 * 4 : 2 * NN * 8;
         const size_t per = 2 * NN * 8 + images + (size_t)p.nLagA * p.nLagR * 4 +
-                           (size_t)p.nLagA * sizeof(RowBest) + 2 * (size_t)(nblk + 1) * 32 +
+                           (size_t)nRun * sizeof(RowBest) + 2 * (size_t)(nblk + 1) * 32 +
                            (size_t)((p.W_A + kTile - 1) / kTile) * 2 * p.W_R * 8 + 4096;
         // a batch the device cannot hold is halved until it fits
         size_t budget = std::max(ctx->scratchBudget, per * 4);
@@ -1057,11 +1109,9 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
         Bt.chip = ar.take<double>(2 * (size_t)B);
         Bt.csum = ar.take<double>((size_t)B * ((p.W_A + kTile - 1) / kTile) * 2 * p.W_R);
         Bt.cr = ar.take<float>((size_t)B * p.nLagA * p.nLagR);
-        Bt.rows = ar.take<RowBest>((size_t)B * p.nLagA);
+        Bt.rows = ar.take<RowBest>((size_t)B * nRun);
         Bt.az = ar.take<int>(B);
-        const int nStep = (int)std::min<size_t>(kNccStep, 65536 / (2 * (size_t)(p.W_R + 1) * sizeof(double)));
-        ST_REQUIRE(nStep >= 1 && p.W_R <= 256 * 8, ST_ERR_UNSUPPORTED, "window too large for the NCC kernel");
-        const size_t ldsNcc = (size_t)nStep * 2 * (p.W_R + 1) * sizeof(double);
+        ST_REQUIRE(p.W_R <= 256 * 8, ST_ERR_UNSUPPORTED, "window too large for the NCC kernel");
         const stfft::PlanArgs PfR = ctx->fft.plan(p.wRa, -1), PiR = ctx->fft.plan(p.W_R, +1);
         const stfft::PlanArgs PfA = ctx->fft.plan(p.wAa, -1), PiA = ctx->fft.plan(p.W_A, +1);
         const size_t ldsRow = (size_t)R * p.W_R * sizeof(float2), ldsCol = (size_t)C * (p.W_A + 1) * sizeof(float2);
@@ -1116,7 +1166,11 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                 });
                 ctx->time_end(kFftSlot);
                 ctx->time_begin(kNcc);
-                hipLaunchKernelGGL((k_w_ncc<4, true>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
+                ncc_size(p.W_R, [&](auto per, auto step) {
+                    if constexpr (per <= 3)  // up to 768 columns
+                        hipLaunchKernelGGL((k_w_ncc<per, step, true>), gNcc, dim3(256),
+                                           step * 2 * (p.W_R + 1) * sizeof(double), st, p, Bt, F, nRun);
+                });
                 ctx->time_end(kNcc);
             } else {
                 ctx->time_begin(kFftSlot);
@@ -1139,14 +1193,14 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                 ctx->fft.fft2d(Bt.U, TMP, np, p.W_A, p.W_R, +1, st);
                 ctx->time_end(kFftSlot);
                 ctx->time_begin(kNcc);
-                if (p.W_R <= 256 * 4)
-                    hipLaunchKernelGGL((k_w_ncc<4, false>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
-                else
-                    hipLaunchKernelGGL((k_w_ncc<8, false>), gNcc, dim3(256), ldsNcc, st, p, Bt, F, nRun, nStep);
+                ncc_size(p.W_R, [&](auto per, auto step) {
+                    hipLaunchKernelGGL((k_w_ncc<per, step, false>), gNcc, dim3(256),
+                                       step * 2 * (p.W_R + 1) * sizeof(double), st, p, Bt, F, nRun);
+                });
                 ctx->time_end(kNcc);
             }
             ctx->time_begin(kRef);
-            hipLaunchKernelGGL(k_w_refine, dim3(nb), dim3(256), 0, st, p, Bt);
+            hipLaunchKernelGGL(k_w_refine, dim3(nb), dim3(256), 0, st, p, Bt, nRun);
             ctx->time_end(kRef);
             ST_HIP(hipGetLastError());
         }

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from specklesource_amd import abi, configs, track
+from tests.test_gpu_strackw import _check, _run, compare
 from tests.test_oracle_strackw import stw_params
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +51,22 @@ def test_equals_general_passes(device, monkeypatch, wr, wa, edge_r, edge_a, navg
     for k in ("offR", "offA", "corr", "type"):
         np.testing.assert_array_equal(getattr(fixed, k), getattr(general, k), err_msg=k)
     assert (fixed.nAmp, fixed.nFail) == (general.nAmp, general.nFail)
+
+
+@pytest.mark.parametrize("wr,edge", [(64, 4), (160, 20), (448, 200), (640, 30), (768, 60), (1024, 500)])
+def test_coarse_correlation_widths(device, oracle32, oracle64, wr, edge):
+    """The column splits of the coarse correlation outside the fixed sizes
+    (1 to 8 columns a thread, 4 to 1 rows a round, a last thread with fewer
+    columns) against the oracle, by the rules of test_gpu_strackw."""
+    na, nr = 160, wr + 120
+    s = configs._spec(nr, na, 11 + wr, dr0=1.7, drR=0.5 / nr, da0=-2.4, daA=3e-3, gmin=0.7, gmax=0.9, gLr=nr / 1.2,
+                      gLa=na / 1.4)
+    par = stw_params(64, nr, na, 8, navg=2, rShiftPoly=[1.7, 0, 0], aShiftPoly=[-2.4, 0, 3e-3], wR=wr, wA=64, wRa=wr,
+                     wAa=64, edgePadR=edge, edgePadA=8, rStart=wr // 2 + 9, aStart=45, deltaR=90, deltaA=60, nR=2, nA=2)
+    a, b = track.synth_host(s)
+    g = _run(device, par, a, b)
+    rep, probs = compare(g, oracle32.corr_track_fast(par, a, b, diag=True),
+                         oracle64.corr_track_fast(par, a, b, diag=True))
+    print("\n", rep)
+    assert rep["patches"] == 4
+    _check(rep, probs)
