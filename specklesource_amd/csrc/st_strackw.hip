@@ -1120,7 +1120,7 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
             const int nb = std::min(B, nList - off);
             const int np = (nb + 1) / 2;
             Bt.res = dRes + off;
-            const dim3 gDet((p.W_R + kTile - 1) / kTile, (p.W_A + kTile - 1) / kTile, nb), gNcc(nRun, nb);
+            const dim3 gNcc(nRun, nb);
             if (fixed) {
                 ctx->time_begin(kFftSlot);
                 wf_size(p.wRa, [&](auto n) {
@@ -1138,7 +1138,7 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                 });
                 ctx->time_end(kFftSlot);
                 ctx->time_begin(kDet);
-                hipLaunchKernelGGL(k_wf_detect, gDet, dim3(256), detect_lds_bytes(p), st, p, Bt, F, nb);
+                launch_wf_detect(p, Bt, F, nb, st);
                 ctx->time_end(kDet);
                 ctx->time_begin(kStat);
                 hipLaunchKernelGGL(k_w_chipstats<true>, dim3(nb), dim3(NT), 0, st, p, Bt, F);
@@ -1180,7 +1180,8 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                                    PfA, PiA);
                 ctx->time_end(kFftSlot);
                 ctx->time_begin(kDet);
-                hipLaunchKernelGGL(k_w_detect, gDet, dim3(256), detect_lds_bytes(p), st, p, Bt, nb);
+                hipLaunchKernelGGL(k_w_detect, dim3((p.W_R + kTile - 1) / kTile, (p.W_A + kTile - 1) / kTile, nb),
+                                   dim3(256), detect_lds_bytes(p), st, p, Bt, nb);
                 ctx->time_end(kDet);
                 ctx->time_begin(kStat);
                 hipLaunchKernelGGL(k_w_chipstats<false>, dim3(nb), dim3(NT), 0, st, p, Bt, F);

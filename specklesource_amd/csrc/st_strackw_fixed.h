@@ -309,70 +309,151 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_lags(WPar p, WfBatch F, 
 }
 
 #pragma clang fp contract(off)
-// detectPatch from the detected images (k_w_detect's boxcar, clamps and sums).
-__global__ void __launch_bounds__(256) k_wf_detect(WPar p, WBatch Bt, WfBatch F, int B)
+constexpr int kDetW = 64;  // columns of a k_wf_detect tile (kTile rows)
+
+// A tile's haloed source from |z|^2 scale: rows clamped to [0, ymax], columns
+// to [0, W_R - 1] (four at a time: segments start at multiples of four, as does
+// W_R, so that a segment lies inside the image or beside it).
+__device__ inline void wf_tile(float *d, const float *U, int W, int y0, int x0, int TH, int TW, int ymax)
 {
-    extern __shared__ float w_det_lds[];
-    __shared__ float sv[kTile][kTile + 1];
-    const int b = blockIdx.z;
-    const size_t NN = (size_t)p.W_A * p.W_R;
-    const float *U1 = F.U + b * NN, *U2 = F.U + ((size_t)B + b) * NN;
-    const bool box = p.navgA > 1 || p.navgR > 1;
-    const int hA = box ? p.navgA : 0, hR = box ? p.navgR : 0;
-    const int y0 = blockIdx.y * kTile, x0 = blockIdx.x * kTile;
-    const int TH = kTile + 2 * hA, TW = kTile + 2 * hR;
-    float *d1 = w_det_lds, *d2 = w_det_lds + TH * TW;
-    const int c0 = p.epA * WOS, c1 = c0 + p.wA2;  // chip rows [c0, c1)
-    const int e0 = p.epR * WOS, e1 = e0 + p.wR2;  // chip cols [e0, e1)
-    const bool chipTile = y0 < c1 && y0 + kTile > c0 && x0 < e1 && x0 + kTile > e0;
-    const int kmaxC = p.epR * WOS + p.wA2 + p.navgA - 1;
-    const int lmaxC = p.epR * WOS + p.wR2 + p.navgR - 1;
-    const int2 cols = wf_chip_cols(p);
-    for (int t = threadIdx.x; t < TH * TW; t += blockDim.x) {
-        const int ty = t / TW, tx = t - (t / TW) * TW;
-        const int y = y0 - hA + ty, x = x0 - hR + tx;
-        d1[t] = U1[(size_t)imin(imax(y, 0), p.W_A - 1) * p.W_R + imin(imax(x, 0), p.W_R - 1)];
-        if (chipTile) {
-            const int ky2 = imin(imin(imax(y, 0), kmaxC), p.W_A - 1), kx2 = imin(imin(imax(x, 0), lmaxC), p.W_R - 1);
-            // columns outside the chip's reach feed no chip cell
-            d2[t] = kx2 >= cols.x && kx2 < cols.y ? U2[(size_t)ky2 * p.W_R + kx2] : 0.f;
+    const int seg = TW / 4;
+    for (int t = threadIdx.x; t < TH * seg; t += 256) {
+        const int ty = t / seg, tx = (t - ty * seg) * 4, x = x0 + tx;
+        const float *row = U + (size_t)imin(imax(y0 + ty, 0), ymax) * W;
+        float4 v;
+        if (x >= 0 && x < W) {
+            v = *(const float4 *)(row + x);
+        } else {
+            const float e = row[x < 0 ? 0 : W - 1];
+            v = make_float4(e, e, e, e);
         }
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < kTile * kTile; t += blockDim.x) {
-        const int oy = t / kTile, ox = t - (t / kTile) * kTile;
-        const int y = y0 + oy, x = x0 + ox;
-        sv[oy][ox] = 0.f;
-        if (y >= p.W_A || x >= p.W_R)
-            continue;
-        float v1 = 0.f;
-        for (int m = -hA; m <= hA; m++)
-            for (int n = -hR; n <= hR; n++)
-                v1 += d1[(oy + hA + m) * TW + ox + hR + n];
-        if (chipTile && y >= c0 && y < c1 && x >= e0 && x < e1) {
-            float v2 = 0.f;
-            for (int m = -hA; m <= hA; m++)
-                for (int n = -hR; n <= hR; n++)
-                    v2 += d2[(oy + hA + m) * TW + ox + hR + n];
-            F.Cf[((size_t)b * p.wA2 + y - c0) * p.wR2 + x - e0] = sqrtf(v2);
-        }
-        const float sr = sqrtf(v1);
-        sv[oy][ox] = sr;
-        F.Sf[b * NN + (size_t)y * p.W_R + x] = sr;
-    }
-    __syncthreads();
-    if (threadIdx.x < kTile && x0 + (int)threadIdx.x < p.W_R) {
-        double a1 = 0.0, a2 = 0.0;
-        for (int oy = 0; oy < kTile; oy++) {
-            const float v = sv[oy][threadIdx.x];
-            a1 += v;
-            a2 += v * v;
-        }
-        double *cs = Bt.csum + ((size_t)b * gridDim.y + blockIdx.y) * 2 * p.W_R + x0 + threadIdx.x;
-        cs[0] = a1;
-        cs[p.W_R] = a2;
+        *(float4 *)(d + ty * TW + tx) = v;
     }
 }
+
+// Boxcar sums of four neighbours from row[0], each in the order of the
+// reference's loops.  H >= 0: both half-widths are H.
+template <int H>
+__device__ inline void wf_box(const float *row, int TW, int hA, int hR, float (&v)[4])
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        v[k] = 0.f;
+    if constexpr (H >= 0) {
+#pragma unroll
+        for (int m = 0; m <= 2 * H; m++) {
+            float w[4 + 2 * H];
+#pragma unroll
+            for (int n = 0; n < 4 + 2 * H; n++)
+                w[n] = row[m * TW + n];
+#pragma unroll
+            for (int n = 0; n <= 2 * H; n++)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    v[k] += w[n + k];
+        }
+    } else {
+        for (int m = 0; m <= 2 * hA; m++) {
+            const float *r = row + m * TW;
+            float w0 = r[0], w1 = r[1], w2 = r[2];
+            for (int n = 0; n <= 2 * hR; n++) {
+                const float w3 = r[n + 3];
+                v[0] += w0;
+                v[1] += w1;
+                v[2] += w2;
+                v[3] += w3;
+                w0 = w1;
+                w1 = w2;
+                w2 = w3;
+            }
+        }
+    }
+}
+
+// detectPatch from the detected images (k_w_detect's boxcar, clamps and sums):
+// tiles of kTile rows by kDetW columns, four neighbouring cells per thread, the
+// chip's cells in a second turn through the same LDS tile.  H: wf_box's, 0 where
+// there is no boxcar.
+//
+// Bound: the (2 h + 1)^2 ordered sums and their LDS reads, which four
+// neighbours share, then the column sums.  576 patches of 768^2, 5 x 5 boxcar:
+// 0.75 ms; 1.87 with one cell per thread and one load per sample.
+template <int H>
+__global__ void __launch_bounds__(256) k_wf_detect(WPar p, WBatch Bt, WfBatch F, int B)
+{
+    extern __shared__ float4 w_det_lds4[];
+    __shared__ float sv[kTile][kDetW + 1];
+    float *d = (float *)w_det_lds4;
+    const int b = blockIdx.z;
+    const size_t NN = (size_t)p.W_A * p.W_R;
+    const int hA = H >= 0 ? H : p.navgA, hR = H >= 0 ? H : p.navgR, hp = (hR + 3) / 4 * 4;
+    const int y0 = blockIdx.y * kTile, x0 = blockIdx.x * kDetW;
+    const int TH = kTile + 2 * hA, TW = kDetW + 2 * hp;
+    wf_tile(d, F.U + b * NN, p.W_R, y0 - hA, x0 - hp, TH, TW, p.W_A - 1);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTile * kDetW / 1024; k++) {
+        const int t = threadIdx.x + 256 * k, oy = t / (kDetW / 4), ox = (t % (kDetW / 4)) * 4;
+        float v[4];
+        wf_box<H>(d + oy * TW + ox + hp - hR, TW, hA, hR, v);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[i] = sqrtf(v[i]);
+            sv[oy][ox + i] = v[i];
+        }
+        *(float4 *)(F.Sf + b * NN + (size_t)(y0 + oy) * p.W_R + x0 + ox) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+    __syncthreads();
+    // column sums of s and of s^2 (FP64) over the tile's rows
+    if (threadIdx.x < 2 * kDetW) {
+        const int c = threadIdx.x % kDetW;
+        const bool sq = threadIdx.x >= kDetW;
+        double a = 0.0;
+        for (int oy = 0; oy < kTile; oy++) {
+            const float v = sv[oy][c];
+            a += sq ? v * v : v;
+        }
+        Bt.csum[(((size_t)b * gridDim.y + blockIdx.y) * 2 + (sq ? 1 : 0)) * p.W_R + x0 + c] = a;
+    }
+    const int c0 = p.epA * WOS, c1 = c0 + p.wA2;  // chip rows [c0, c1)
+    const int e0 = p.epR * WOS, e1 = e0 + p.wR2;  // chip cols [e0, e1)
+    if (y0 >= c1 || y0 + kTile <= c0 || x0 >= e1 || x0 + kDetW <= e0)
+        return;
+    // the azimuth clamp is the reference's, written with the range pad; the
+    // columns that k_wf_cols left out reach no cell of the chip
+    const int kmaxC = imin(p.epR * WOS + p.wA2 + p.navgA - 1, p.W_A - 1);
+    wf_tile(d, F.U + ((size_t)B + b) * NN, p.W_R, y0 - hA, x0 - hp, TH, TW, kmaxC);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTile * kDetW / 1024; k++) {
+        const int t = threadIdx.x + 256 * k, oy = t / (kDetW / 4), ox = (t % (kDetW / 4)) * 4;
+        const int y = y0 + oy, x = x0 + ox;
+        if (y < c0 || y >= c1 || x + 3 < e0 || x >= e1)
+            continue;
+        float v[4];
+        wf_box<H>(d + oy * TW + ox + hp - hR, TW, hA, hR, v);
+        float *c = F.Cf + ((size_t)b * p.wA2 + y - c0) * p.wR2 - e0 + x;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (x + i >= e0 && x + i < e1)
+                c[i] = sqrtf(v[i]);
+    }
+}
+
+inline void launch_wf_detect(const WPar &p, const WBatch &Bt, const WfBatch &F, int nb, hipStream_t st)
+{
+    const bool box = p.navgA > 1 || p.navgR > 1;  // detectPatch's test
+    const int hA = box ? p.navgA : 0, hR = box ? p.navgR : 0;
+    const size_t lds = (size_t)(kTile + 2 * hA) * (kDetW + (hR + 3) / 4 * 8) * sizeof(float);
+    const dim3 g(p.W_R / kDetW, p.W_A / kTile, nb);
+    if (!box)
+        hipLaunchKernelGGL(k_wf_detect<0>, g, dim3(256), lds, st, p, Bt, F, nb);
+    else if (hA == 2 && hR == 2)  // the trackers' own boxcar
+        hipLaunchKernelGGL(k_wf_detect<2>, g, dim3(256), lds, st, p, Bt, F, nb);
+    else
+        hipLaunchKernelGGL(k_wf_detect<-1>, g, dim3(256), lds, st, p, Bt, F, nb);
+}
+
 // S conj(C) at a frequency from Z there (a) and at its mirror (c): k_w_cross's
 // expressions.
 __device__ inline float2 wf_cross(float2 a, float2 c)
