@@ -22,13 +22,15 @@ struct Plan {
 
 inline bool covered(int n) { return n == 128 || n == 192 || n == 256 || n == 384; }
 
-template <int N>
-__device__ inline float2 twiddle(int e)  // exp(-2 pi i e / N)
+// Fills tw[e] = exp(-2 pi i e / L), e < L, by all threads of a workgroup (a
+// barrier follows before its use).  The stages read their twiddles from there:
+// a lane's own values come from up to 64 places of the table, which LDS serves
+// several times as fast as the vector caches do.
+template <int L>
+__device__ inline void table(float2 *tw)
 {
-    if constexpr (N % 3 == 0)
-        return c_tw768[e * (768 / N)];
-    else
-        return c_tw512[e * (512 / N)];
+    for (int e = threadIdx.x; e < L; e += blockDim.x)
+        tw[e] = L % 3 ? c_tw512[e * (512 / L)] : c_tw768[e * (768 / L)];
 }
 
 template <int SIGN>
@@ -44,18 +46,20 @@ __device__ inline void dft3(float2 &a, float2 &b, float2 &d)
 }
 
 // One stage: butterflies jj = j + LANES u, u < V / R, on elements u + (V / R) r.
-template <int N, int R, int NS, int SIGN>
-__device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex)
+template <int N, int R, int NS, int SIGN, int L>
+__device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex, const float2 *tw)
 {
     constexpr int V = Plan<N>::V, LANES = Plan<N>::LANES, NB = V / R;
     static_assert(NB * R == V, "radix divides the lane's values");
+    // opaque: no stage's addresses are computed ahead and held in registers
+    asm volatile("" : "+v"(j));
 #pragma unroll
     for (int u = 0; u < NB; u++) {
         const int k = (j + LANES * u) % NS;
         if constexpr (NS > 1) {
 #pragma unroll
             for (int r = 1; r < R; r++)
-                v[u + NB * r] = fft8::mul_tw<SIGN>(v[u + NB * r], twiddle<N>(k * r * (N / (NS * R))));
+                v[u + NB * r] = fft8::mul_tw<SIGN>(v[u + NB * r], tw[k * r * (L / (NS * R))]);
         }
         if constexpr (R == 8) {
             float2 w[8];
@@ -72,7 +76,20 @@ __device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex)
             dft3<SIGN>(v[u], v[u + NB], v[u + 2 * NB]);
         }
     }
-    if constexpr (NS * R < N) {
+    if constexpr (NS * R < N && NS % LANES == 0) {
+        // the next stage's inputs are the lane's own: element j + LANES i moves
+        // to another i
+        constexpr int S = NS / LANES;
+        float2 w[V];
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+#pragma unroll
+            for (int q = 0; q < R; q++)
+                w[(u / S) * S * R + u % S + S * q] = v[u + NB * q];
+#pragma unroll
+        for (int i = 0; i < V; i++)
+            v[i] = w[i];
+    } else if constexpr (NS * R < N) {
 #pragma unroll
         for (int u = 0; u < NB; u++) {
             const int jj = j + LANES * u, at = (jj / NS) * NS * R + jj % NS;
@@ -88,30 +105,32 @@ __device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex)
     }
 }
 
-template <int N, int SIGN>
-__device__ inline void fft(float2 (&v)[Plan<N>::V], int j, float2 *ex)
+// tw: table<L>, L a multiple of N.
+template <int N, int SIGN, int L>
+__device__ inline void fft(float2 (&v)[Plan<N>::V], int j, float2 *ex, const float2 *tw)
 {
-    stage<N, 8, 1, SIGN>(v, j, ex);
+    static_assert(L % N == 0, "table of twiddles");
+    stage<N, 8, 1, SIGN, L>(v, j, ex, tw);
     if constexpr (N == 128) {
-        stage<N, 4, 8, SIGN>(v, j, ex);
-        stage<N, 4, 32, SIGN>(v, j, ex);
+        stage<N, 4, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 4, 32, SIGN, L>(v, j, ex, tw);
     } else if constexpr (N == 192) {
-        stage<N, 8, 8, SIGN>(v, j, ex);
-        stage<N, 3, 64, SIGN>(v, j, ex);
+        stage<N, 8, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 3, 64, SIGN, L>(v, j, ex, tw);
     } else if constexpr (N == 256) {
-        stage<N, 8, 8, SIGN>(v, j, ex);
-        stage<N, 4, 64, SIGN>(v, j, ex);
+        stage<N, 8, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 4, 64, SIGN, L>(v, j, ex, tw);
     } else if constexpr (N == 384) {
-        stage<N, 4, 8, SIGN>(v, j, ex);
-        stage<N, 4, 32, SIGN>(v, j, ex);
-        stage<N, 3, 128, SIGN>(v, j, ex);
+        stage<N, 4, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 4, 32, SIGN, L>(v, j, ex, tw);
+        stage<N, 3, 128, SIGN, L>(v, j, ex, tw);
     } else if constexpr (N == 512) {
-        stage<N, 8, 8, SIGN>(v, j, ex);
-        stage<N, 8, 64, SIGN>(v, j, ex);
+        stage<N, 8, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 8, 64, SIGN, L>(v, j, ex, tw);
     } else {
-        stage<N, 8, 8, SIGN>(v, j, ex);
-        stage<N, 4, 64, SIGN>(v, j, ex);
-        stage<N, 3, 256, SIGN>(v, j, ex);
+        stage<N, 8, 8, SIGN, L>(v, j, ex, tw);
+        stage<N, 4, 64, SIGN, L>(v, j, ex, tw);
+        stage<N, 3, 256, SIGN, L>(v, j, ex, tw);
     }
 }
 

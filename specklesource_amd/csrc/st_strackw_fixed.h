@@ -30,13 +30,22 @@ template <int N>
 struct WfGeom {
     static constexpr int M = 2 * N, VN = fftn::Plan<N>::V, LN = fftn::Plan<N>::LANES;
     static constexpr int VM = fftn::Plan<M>::V, LM = fftn::Plan<M>::LANES;
-    // an LDS region: N + N / 8 elements, 8 more than a multiple of 32 so that
+    // LDS: the twiddle table (M elements), then a region per row or column of
+    // M + M / 8 elements and some, 8 more than a multiple of 32 so that
     // stores and loads of 8 columns across 8 regions meet no bank twice
     static constexpr int PB = (M + M / 8 + 23) / 32 * 32 + 8;
     static constexpr int R = 256 / LM, NTHR = R * LM;
     static constexpr int C = 8, NTHC = C * LM;
-    static constexpr size_t LDSR = (size_t)R * PB * sizeof(float2), LDSC = (size_t)C * PB * sizeof(float2);
+    static constexpr size_t LDSR = (size_t)(M + R * PB) * sizeof(float2), LDSC = (size_t)(M + C * PB) * sizeof(float2);
     static_assert(LM == 2 * LN && VM == VN, "lane groups");
+    // start of lane group g's exchanges: regions start 8 banks apart, which
+    // keeps groups of 8 lanes off each other's banks, groups of 16 lanes need 16
+    template <int LANES>
+    __device__ static inline int at(int g)
+    {
+        return g * PB + (LANES == 16 ? (g & 1) * 8 : 0);
+    }
+    static_assert(PB >= M + M / 8 + (LM == 16 ? 8 : 0), "room for the shift");
 };
 
 struct WfBatch {
@@ -62,17 +71,17 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
 {
     using G = WfGeom<N>;
     constexpr int V = G::VN, NW = G::NTHR / 64;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     __shared__ double sh[NW][4];
     const int z = blockIdx.y, img = z >= B ? 1 : 0, b = z - img * B, t = threadIdx.x;
     const int4 q = Bt.pos[off + b];
     const int rr = img ? q.z : q.x, ra = img ? q.w : q.y;
     const int i0 = blockIdx.x * G::R;
     double s[4] = {0, 0, 0, 0};  // sum x, sum x[i + 1] conj(x[i]) (re, im)
+    float2 v[V];
     if (t < G::R * G::LN) {
         const int j = t % G::LN, i = i0 + t / G::LN;
-        float2 *ex = ldsf + (t / G::LN) * G::PB;
-        float2 v[V];
         const bool next = i + 1 < p.wAa;
 #pragma unroll
         for (int r = 0; r < V; r++)
@@ -102,7 +111,13 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
                 s[2] += (double)x1.x * x0.x + (double)x1.y * x0.y;
                 s[3] += (double)x1.y * x0.x - (double)x1.x * x0.y;
             }
-        fftn::fft<N, -1>(v, j, ex);
+    }
+    fftn::table<G::M>(tw);
+    __syncthreads();
+    if (t < G::R * G::LN) {
+        const int j = t % G::LN;
+        float2 *ex = ldsf + G::template at<G::LN>(t / G::LN);
+        fftn::fft<N, -1, G::M>(v, j, ex, tw);
 #pragma unroll
         for (int r = 0; r < V; r++)
             ex[j + G::LN * r] = v[r];
@@ -123,17 +138,16 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
         Bt.dop[((size_t)z * gridDim.x + blockIdx.x) * 4 + t] = a;
     }
     const int j = t % G::LM, i = i0 + t / G::LM;
-    float2 *ex = ldsf + (t / G::LM) * G::PB;
-    float2 v[V];
+    const float2 *in = ldsf + G::template at<G::LN>(t / G::LM);
 #pragma unroll
     for (int r = 0; r < V; r++) {
         // bins 0 .. N / 2 - 1 stay, the Nyquist bin and the negative
         // frequencies move to the top, zeros between
         const int m = j + G::LM * r;
-        v[r] = r < V / 4 ? ex[m] : r >= V - V / 4 ? ex[m - N] : make_float2(0.f, 0.f);
+        v[r] = r < V / 4 ? in[m] : r >= V - V / 4 ? in[m - N] : make_float2(0.f, 0.f);
     }
     fft8::wave_sync();
-    fftn::fft<G::M, +1>(v, j, ex);
+    fftn::fft<G::M, +1, G::M>(v, j, ldsf + G::template at<G::LM>(t / G::LM), tw);
     const int2 cols = img ? wf_chip_cols(p) : make_int2(0, p.W_R);
     float2 *T = Bt.T + ((size_t)z * p.wAa + i) * p.W_R;
 #pragma unroll
@@ -151,7 +165,8 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
 {
     using G = WfGeom<N>;
     constexpr int V = G::VN, C = G::C, M = G::M, LM = G::LM, LN = G::LN;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
     const int L = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;  // neighbouring column blocks on one XCD
     const int b = L / nbx, blk = L - b * nbx, img = blk >= nb0 ? 1 : 0, z = img * B + b, t = threadIdx.x;
@@ -159,24 +174,27 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
     const float2 *T = Bt.T + (size_t)z * p.wAa * p.W_R + c0;
     {
         constexpr int K = N / LM;
+        const unsigned at = (t / C) * p.W_R + t % C;  // beside a uniform base
         float2 u[K];
 #pragma unroll
         for (int k = 0; k < K; k++)
-            u[k] = T[(size_t)(t / C + k * LM) * p.W_R + t % C];
+            u[k] = (T + (size_t)(k * LM) * p.W_R)[at];
 #pragma unroll
         for (int k = 0; k < K; k++)
             ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
     }
+    fftn::table<G::M>(tw);
     __syncthreads();
     if (t < C * LN) {
         const int j = t % LN;
-        float2 *ex = ldsf + (t / LN) * G::PB;
+        const float2 *in = ldsf + (t / LN) * G::PB;
+        float2 *ex = ldsf + G::template at<LN>(t / LN);
         float2 v[V];
 #pragma unroll
         for (int r = 0; r < V; r++)
-            v[r] = ex[j + LN * r];
+            v[r] = in[j + LN * r];
         fft8::wave_sync();
-        fftn::fft<N, -1>(v, j, ex);
+        fftn::fft<N, -1, G::M>(v, j, ex, tw);
 #pragma unroll
         for (int r = 0; r < V; r++)
             ex[j + LN * r] = v[r];
@@ -184,7 +202,8 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
     __syncthreads();
     {
         const int j = t % LM, az = Bt.az[b];
-        float2 *ex = ldsf + (t / LM) * G::PB;
+        const float2 *in = ldsf + G::template at<LN>(t / LM);
+        float2 *ex = ldsf + G::template at<LM>(t / LM);
         float2 v[V];
 #pragma unroll
         for (int r = 0; r < V; r++) {
@@ -192,12 +211,12 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
             if (r < V / 4 || r >= V - V / 4) {
                 int k = j + LM * r + (r < V / 4 ? 0 : N - M) + az;  // in [0, 2 N)
                 k -= k >= N ? N : 0;
-                v[r] = ex[k];
+                v[r] = in[k];
             }
         }
         fft8::wave_sync();
-        fftn::fft<M, +1>(v, j, ex);
-        float *exf = (float *)ex;
+        fftn::fft<M, +1, G::M>(v, j, ex, tw);
+        float *exf = (float *)(ldsf + (t / LM) * G::PB);
 #pragma unroll
         for (int r = 0; r < V; r++) {
 #pragma clang fp contract(off)
@@ -206,11 +225,10 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
     }
     __syncthreads();
     float *U = F.U + (size_t)z * p.W_A * p.W_R + c0;
+    const unsigned at = (t / C) * p.W_R + t % C;
 #pragma unroll
-    for (int k = 0; k < M / LM; k++) {
-        const int n = t / C + k * LM;
-        U[(size_t)n * p.W_R + t % C] = ((const float *)(ldsf + (t % C) * G::PB))[n];
-    }
+    for (int k = 0; k < M / LM; k++)
+        (U + (size_t)(k * LM) * p.W_R)[at] = ((const float *)(ldsf + (t % C) * G::PB))[t / C + k * LM];
 }
 
 template <int N>
@@ -218,7 +236,8 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_zrows(WPar p, WBatch Bt,
 {
     using G = WfGeom<N>;
     constexpr int V = G::VM, LM = G::LM;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     const int b = blockIdx.y, t = threadIdx.x, j = t % LM, y = blockIdx.x * G::R + t / LM;
     const float *S = F.Sf + ((size_t)b * p.W_A + y) * p.W_R + j;
     const int yc = y - p.epA * WOS, e0 = p.epR * WOS;
@@ -230,7 +249,9 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_zrows(WPar p, WBatch Bt,
         const int x = j + LM * r;
         v[r] = make_float2(S[LM * r], in && x >= e0 && x < e0 + p.wR2 ? Cr[LM * r] : 0.f);
     }
-    fftn::fft<G::M, -1>(v, j, ldsf + (t / LM) * G::PB);
+    fftn::table<G::M>(tw);
+    __syncthreads();
+    fftn::fft<G::M, -1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
     float2 *Z = Bt.Zs + ((size_t)b * p.W_A + y) * p.W_R + j;
 #pragma unroll
     for (int r = 0; r < V; r++)
@@ -242,14 +263,17 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_urows(WPar p, WfBatch F)
 {
     using G = WfGeom<N>;
     constexpr int V = G::VM, M = G::M, LM = G::LM;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     const int q = blockIdx.y, t = threadIdx.x, j = t % LM, y = blockIdx.x * G::R + t / LM;
     const float2 *Gq = F.G + ((size_t)q * p.W_A + y) * p.W_R + j;
     float2 v[V];
 #pragma unroll
     for (int r = 0; r < V; r++)
         v[r] = Gq[LM * r];
-    fftn::fft<M, +1>(v, j, ldsf + (t / LM) * G::PB);
+    fftn::table<G::M>(tw);
+    __syncthreads();
+    fftn::fft<M, +1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
     const int lagR = WOS * p.epR;
     float2 *X = F.X + ((size_t)q * p.W_A + y) * F.pitchX;
 #pragma unroll
@@ -267,7 +291,8 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_lags(WPar p, WfBatch F, 
 {
     using G = WfGeom<N>;
     constexpr int V = G::VM, C = G::C, M = G::M, LM = G::LM;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
     const int L = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;
     const int q = L / nbx, c0 = (L - q * nbx) * C, t = threadIdx.x, j = t % LM;
@@ -275,20 +300,23 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_lags(WPar p, WfBatch F, 
     float2 *ex = ldsf + (t / LM) * G::PB;
     {
         float2 u[M / LM];
+        const unsigned at = (t / C) * F.pitchX + t % C;
 #pragma unroll
         for (int k = 0; k < M / LM; k++)
-            u[k] = X[(size_t)(t / C + k * LM) * F.pitchX + t % C];
+            u[k] = (X + (size_t)(k * LM) * F.pitchX)[at];
 #pragma unroll
         for (int k = 0; k < M / LM; k++)
             ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
     }
+    fftn::table<G::M>(tw);
     __syncthreads();
     float2 v[V];
 #pragma unroll
     for (int r = 0; r < V; r++)
         v[r] = ex[j + LM * r];
     fft8::wave_sync();
-    fftn::fft<M, +1>(v, j, ex);
+    fftn::fft<M, +1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
+    fft8::wave_sync();
 #pragma unroll
     for (int r = 0; r < V; r++)
         ex[j + LM * r] = v[r];
@@ -472,13 +500,15 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch 
 {
     using G = WfGeom<N>;
     constexpr int V = G::VM, C = G::C, M = G::M, LM = G::LM;
-    extern __shared__ float2 ldsf[];
+    extern __shared__ float2 tw[];
+    float2 *ldsf = tw + G::M;
     const int nbx = gridDim.x, total = nbx * gridDim.y, flat = blockIdx.y * nbx + blockIdx.x, per = total / 8;
     const int Lb = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;
     const int q = Lb / nbx, c0 = (Lb - q * nbx) * C, t = threadIdx.x, W = p.W_R, H = W / 2;
     const int j = t % LM, slot = t / LM;
-    float2 *ex = ldsf + slot * G::PB;
+    float2 *ex = ldsf + slot * G::PB, *sx = ldsf + G::template at<LM>(slot);
     const bool self = c0 + slot == 0;
+    fftn::table<G::M>(tw);
     // column of load / store lane t % C on side s (0: l, 1: mirror)
     auto col = [&](int s) {
         const int l = c0 + t % C;
@@ -486,10 +516,10 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch 
     };
     auto load = [&](const float2 *Z, int s, float2(&v)[V]) {
         float2 u[M / LM];
-        const int c = col(s);
+        const unsigned at = (t / C) * W + col(s);
 #pragma unroll
         for (int k = 0; k < M / LM; k++)
-            u[k] = Z[(size_t)(t / C + k * LM) * W + c];
+            u[k] = (Z + (size_t)(k * LM) * W)[at];
         __syncthreads();  // the region's last readers are done
 #pragma unroll
         for (int k = 0; k < M / LM; k++)
@@ -505,9 +535,13 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch 
         const float2 *Z = Bt.Zs + (size_t)(2 * q + h) * p.W_A * W;
         float2 x[V], y[V];
         load(Z, 0, x);
-        fftn::fft<M, -1>(x, j, ex);
+        __builtin_amdgcn_sched_barrier(0);
+        fftn::fft<M, -1, G::M>(x, j, sx, tw);
+        __builtin_amdgcn_sched_barrier(0);
         load(Z, 1, y);
-        fftn::fft<M, -1>(y, j, ex);
+        __builtin_amdgcn_sched_barrier(0);
+        fftn::fft<M, -1, G::M>(y, j, sx, tw);
+        __builtin_amdgcn_sched_barrier(0);
         // side s: the region takes the column at -l (columns 0 and W_R / 2 are their own)
         auto side = [&](auto s) {
             float2(&m)[V] = s == 0 ? x : y;
@@ -535,12 +569,10 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch 
         for (int r = 0; r < V; r++)
             ex[j + LM * r] = g[s][r];
         __syncthreads();
-        const int c = col(s);
+        const unsigned at = (t / C) * W + col(s);
 #pragma unroll
-        for (int k = 0; k < M / LM; k++) {
-            const int n = t / C + k * LM;
-            Gq[(size_t)n * W + c] = ldsf[(t % C) * G::PB + n];
-        }
+        for (int k = 0; k < M / LM; k++)
+            (Gq + (size_t)(k * LM) * W)[at] = ldsf[(t % C) * G::PB + t / C + k * LM];
         __syncthreads();
     }
 }
