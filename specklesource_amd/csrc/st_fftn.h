@@ -46,8 +46,8 @@ __device__ inline void dft3(float2 &a, float2 &b, float2 &d)
 }
 
 // One stage: butterflies jj = j + LANES u, u < V / R, on elements u + (V / R) r.
-template <int N, int R, int NS, int SIGN, int L>
-__device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex, const float2 *tw)
+template <int N, int R, int NS, int SIGN, int L, class EX>
+__device__ inline void stage(float2 (&v)[Plan<N>::V], int j, EX *ex, const float2 *tw)
 {
     constexpr int V = Plan<N>::V, LANES = Plan<N>::LANES, NB = V / R;
     static_assert(NB * R == V, "radix divides the lane's values");
@@ -90,24 +90,37 @@ __device__ inline void stage(float2 (&v)[Plan<N>::V], int j, float2 *ex, const f
         for (int i = 0; i < V; i++)
             v[i] = w[i];
     } else if constexpr (NS * R < N) {
+        // float2 regions take both parts at once, float ones the real parts, then the imaginary
+        constexpr int PARTS = sizeof(EX) == sizeof(float2) ? 1 : 2;
 #pragma unroll
-        for (int u = 0; u < NB; u++) {
-            const int jj = j + LANES * u, at = (jj / NS) * NS * R + jj % NS;
+        for (int p = 0; p < PARTS; p++) {
 #pragma unroll
-            for (int q = 0; q < R; q++)
-                ex[fft8::pad(at + q * NS)] = v[u + NB * q];
+            for (int u = 0; u < NB; u++) {
+                const int jj = j + LANES * u, at = (jj / NS) * NS * R + jj % NS;
+#pragma unroll
+                for (int q = 0; q < R; q++) {
+                    if constexpr (PARTS == 1)
+                        ex[fft8::pad(at + q * NS)] = v[u + NB * q];
+                    else
+                        ex[fft8::pad(at + q * NS)] = p == 0 ? v[u + NB * q].x : v[u + NB * q].y;
+                }
+            }
+            fft8::wave_sync();
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                if constexpr (PARTS == 1)
+                    v[i] = ex[fft8::pad(j + LANES * i)];
+                else
+                    (p == 0 ? v[i].x : v[i].y) = ex[fft8::pad(j + LANES * i)];
+            }
+            fft8::wave_sync();
         }
-        fft8::wave_sync();
-#pragma unroll
-        for (int i = 0; i < V; i++)
-            v[i] = ex[fft8::pad(j + LANES * i)];
-        fft8::wave_sync();
     }
 }
 
 // tw: table<L>, L a multiple of N.
-template <int N, int SIGN, int L>
-__device__ inline void fft(float2 (&v)[Plan<N>::V], int j, float2 *ex, const float2 *tw)
+template <int N, int SIGN, int L, class EX>
+__device__ inline void fft(float2 (&v)[Plan<N>::V], int j, EX *ex, const float2 *tw)
 {
     static_assert(L % N == 0, "table of twiddles");
     stage<N, 8, 1, SIGN, L>(v, j, ex, tw);

@@ -1046,8 +1046,8 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
     if (nList > 0) {
         const size_t NN = (size_t)p.W_A * p.W_R;
         // The fixed-size passes take the sizes they are built for: there they
-        // beat the general ones (750 points of 128^2 windows 2.58 -> 1.84 ms,
-        // 576 of 384^2 18.6 -> 11.8 ms); the general ones stay for all others,
+        // beat the general ones (whole tracker, 750 points of 128^2 windows 2.2 ->
+        // 1.17 ms, 576 of 384^2 17.3 -> 7.5 ms); the general ones stay for all others,
         // and on request.
         const char *path = getenv("SPECKLE_AMD_PATH");
         const bool fixed = wf_covered(p) && !(path && strcmp(path, "staged") == 0);
@@ -1151,7 +1151,7 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                 });
                 wf_size(p.wAa, [&](auto n) {
                     using G = WfGeom<decltype(n)::value>;
-                    hipLaunchKernelGGL(k_wf_cross<decltype(n)::value>, dim3(p.W_R / 2 / G::C, np), dim3(G::NTHC), G::LDSC,
+                    hipLaunchKernelGGL(k_wf_cross<decltype(n)::value>, dim3(p.W_R / 2 / G::C, np), dim3(G::NTHC), G::LDSF,
                                        st, p, Bt, F, nb);
                 });
                 wf_size(p.wRa, [&](auto n) {
@@ -1162,7 +1162,7 @@ void st_corr_track_fast_impl(st_ctx *ctx, StPair &pr, const st_track_params &par
                 wf_size(p.wAa, [&](auto n) {
                     using G = WfGeom<decltype(n)::value>;
                     hipLaunchKernelGGL(k_wf_lags<decltype(n)::value>, dim3((p.nLagR + G::C - 1) / G::C, np),
-                                       dim3(G::NTHC), G::LDSC, st, p, F, nb);
+                                       dim3(G::NTHC), G::LDSF, st, p, F, nb);
                 });
                 ctx->time_end(kFftSlot);
                 ctx->time_begin(kNcc);

@@ -18,11 +18,10 @@
 // Values stay in registers between the stages of a transform and images are
 // stored as floats, of the chip only what is read; the general passes exchange
 // every stage through LDS with a block barrier and move complex images.  576
-// windows of 384^2, general -> here: interpolation 6.6 -> 3.2 ms, detection
-// 2.04 -> 1.87, chip statistics 0.16 -> 0.12, correlation transforms with the
-// cross spectra 7.0 -> 4.0, coarse correlation 2.60 -> 2.43.  Bound: LDS
-// exchanges and VALU issue at two waves per SIMD in the interpolation and the
-// cross spectra, HBM in k_wf_zrows, k_wf_urows and k_wf_lags (3.4 to 4.9 TB/s).
+// windows of 384^2, general -> here: interpolation 6.6 -> 2.3 ms, detection
+// 2.04 -> 0.79, correlation transforms with the cross spectra 7.0 -> 3.0.
+// k_wf_zrows, k_wf_urows and k_wf_lags run at 3.7 to 5.4 TB/s, the cross spectra
+// at 3.3, the interpolation at 2.8 with LDS and VALU issue beside it.
 
 // Geometry for window side N: M = 2 N interpolated samples, C columns (or
 // slots) and R rows per workgroup.
@@ -30,22 +29,42 @@ template <int N>
 struct WfGeom {
     static constexpr int M = 2 * N, VN = fftn::Plan<N>::V, LN = fftn::Plan<N>::LANES;
     static constexpr int VM = fftn::Plan<M>::V, LM = fftn::Plan<M>::LANES;
-    // LDS: the twiddle table (M elements), then a region per row or column of
-    // M + M / 8 elements and some, 8 more than a multiple of 32 so that
-    // stores and loads of 8 columns across 8 regions meet no bank twice
+    // LDS: the twiddle table (M elements), then a region per row or column.
+    // Full regions hold M + M / 8 complex elements and some: 8 more than a
+    // multiple of 32, so that stores and loads of 8 columns across 8 regions meet
+    // no bank twice.  Where a lane holds 24 values (a third of the lanes that 8
+    // take) full regions would leave two waves per SIMD: there the kernels that
+    // can exchange real and imaginary parts in turn (half regions: M + M / 8
+    // floats and some, 8 more than a multiple of 64).
     static constexpr int PB = (M + M / 8 + 23) / 32 * 32 + 8;
+    static constexpr bool HALF = VM == 24;
+    static constexpr int PF = HALF ? (M + M / 8 + 24 + 55) / 64 * 64 + 8 : 2 * PB;  // floats
+    using Ex = std::conditional_t<HALF, float, float2>;
     static constexpr int R = 256 / LM, NTHR = R * LM;
     static constexpr int C = 8, NTHC = C * LM;
-    static constexpr size_t LDSR = (size_t)(M + R * PB) * sizeof(float2), LDSC = (size_t)(M + C * PB) * sizeof(float2);
+    static constexpr size_t TW = M * sizeof(float2);
+    static constexpr size_t LDSR = TW + (size_t)R * PF * sizeof(float), LDSC = TW + (size_t)C * PF * sizeof(float);
+    static constexpr size_t LDSF = TW + (size_t)C * PB * sizeof(float2);
     static_assert(LM == 2 * LN && VM == VN, "lane groups");
-    // start of lane group g's exchanges: regions start 8 banks apart, which
-    // keeps groups of 8 lanes off each other's banks, groups of 16 lanes need 16
+    // start of lane group g's exchanges.  Full regions start 8 elements of 32
+    // apart, which keeps groups of 8 lanes off each other's banks: groups of 16
+    // need 16.  Half regions start 8 floats apart and need as much as the group
+    // has lanes.
     template <int LANES>
-    __device__ static inline int at(int g)
+    __device__ static inline float2 *full(float2 *lds, int g)
     {
-        return g * PB + (LANES == 16 ? (g & 1) * 8 : 0);
+        return lds + g * PB + (LANES == 16 ? (g & 1) * 8 : 0);
     }
-    static_assert(PB >= M + M / 8 + (LM == 16 ? 8 : 0), "room for the shift");
+    template <int LANES>
+    __device__ static inline Ex *ex(float2 *lds, int g)
+    {
+        if constexpr (HALF)
+            return (float *)lds + g * PF + (LANES == 32 ? (g & 1) * 24 : LANES == 16 ? (g & 3) * 8 : 0);
+        else
+            return full<LANES>(lds, g);
+    }
+    __device__ static inline float2 *region(float2 *lds, int g) { return lds + g * (PF / 2); }
+    static_assert(PB >= M + M / 8 + (LM == 16 ? 8 : 0) && PF >= M + M / 8 + (HALF ? 24 : 0), "room for the shift");
 };
 
 struct WfBatch {
@@ -66,8 +85,34 @@ __host__ __device__ inline int2 wf_chip_cols(const WPar &p)
     return make_int2(imax(0, e0 - h), imin(p.W_R, e0 + p.wR2 + h));
 }
 
+// A lane's samples r + LN k of image row a.
 template <int N>
-__global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WBatch Bt, int B)
+__device__ inline void wf_samples(const Images &im, int img, int a, int r, bool inside, float2 (&v)[WfGeom<N>::VN])
+{
+    constexpr int V = WfGeom<N>::VN, LN = WfGeom<N>::LN;
+    if (inside) {
+        const size_t o = (size_t)a * (img ? im.nr2 : im.nr1) + r;
+        const void *d = img ? im.img2 : im.img1;
+        if (im.stype == ST_SAMPLE_C64) {
+#pragma unroll
+            for (int k = 0; k < V; k++)
+                v[k] = ((const float2 *)d + o)[LN * k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < V; k++) {
+                const short2 s = ((const short2 *)d + o)[LN * k];
+                v[k] = make_float2((float)s.x, (float)s.y);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < V; k++)
+            v[k] = sample0(im, img, a, r + LN * k);
+    }
+}
+
+template <int N>
+__global__ void __launch_bounds__(WfGeom<N>::NTHR, 4) k_wf_rows(WPar p, int off, WBatch Bt, int B)
 {
     using G = WfGeom<N>;
     constexpr int V = G::VN, NW = G::NTHR / 64;
@@ -78,14 +123,15 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
     const int4 q = Bt.pos[off + b];
     const int rr = img ? q.z : q.x, ra = img ? q.w : q.y;
     const int i0 = blockIdx.x * G::R;
+    // the rows here and the next one inside the image: no tests per sample
+    const int nr = img ? p.im.nr2 : p.im.nr1, na = img ? p.im.na2 : p.im.na1;
+    const bool inside = rr >= 0 && rr + N <= nr && ra + i0 >= 0 && ra + i0 + G::R < na;
     double s[4] = {0, 0, 0, 0};  // sum x, sum x[i + 1] conj(x[i]) (re, im)
     float2 v[V];
     if (t < G::R * G::LN) {
         const int j = t % G::LN, i = i0 + t / G::LN;
         const bool next = i + 1 < p.wAa;
-#pragma unroll
-        for (int r = 0; r < V; r++)
-            v[r] = sample0(p.im, img, ra + i, rr + j + G::LN * r);
+        wf_samples<N>(p.im, img, ra + i, rr + j, inside, v);
 #pragma unroll
         for (int r = 0; r < V; r++) {
             s[0] += v[r].x;
@@ -104,23 +150,26 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
                 E[1] = e1;
             }
         }
-        if (next)
+        if (next) {
+            float2 w[V];
+            wf_samples<N>(p.im, img, ra + i + 1, rr + j, inside, w);
 #pragma unroll
             for (int r = 0; r < V; r++) {
-                const float2 x1 = sample0(p.im, img, ra + i + 1, rr + j + G::LN * r), x0 = v[r];
+                const float2 x1 = w[r], x0 = v[r];
                 s[2] += (double)x1.x * x0.x + (double)x1.y * x0.y;
                 s[3] += (double)x1.y * x0.x - (double)x1.x * x0.y;
             }
+        }
     }
     fftn::table<G::M>(tw);
     __syncthreads();
     if (t < G::R * G::LN) {
         const int j = t % G::LN;
-        float2 *ex = ldsf + G::template at<G::LN>(t / G::LN);
-        fftn::fft<N, -1, G::M>(v, j, ex, tw);
+        float2 *out = G::region(ldsf, t / G::LN);
+        fftn::fft<N, -1, G::M>(v, j, G::template ex<G::LN>(ldsf, t / G::LN), tw);
 #pragma unroll
         for (int r = 0; r < V; r++)
-            ex[j + G::LN * r] = v[r];
+            out[j + G::LN * r] = v[r];
     }
     for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
@@ -138,7 +187,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
         Bt.dop[((size_t)z * gridDim.x + blockIdx.x) * 4 + t] = a;
     }
     const int j = t % G::LM, i = i0 + t / G::LM;
-    const float2 *in = ldsf + G::template at<G::LN>(t / G::LM);
+    const float2 *in = G::region(ldsf, t / G::LM);
 #pragma unroll
     for (int r = 0; r < V; r++) {
         // bins 0 .. N / 2 - 1 stay, the Nyquist bin and the negative
@@ -147,7 +196,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_rows(WPar p, int off, WB
         v[r] = r < V / 4 ? in[m] : r >= V - V / 4 ? in[m - N] : make_float2(0.f, 0.f);
     }
     fft8::wave_sync();
-    fftn::fft<G::M, +1, G::M>(v, j, ldsf + G::template at<G::LM>(t / G::LM), tw);
+    fftn::fft<G::M, +1, G::M>(v, j, G::template ex<G::LM>(ldsf, t / G::LM), tw);
     const int2 cols = img ? wf_chip_cols(p) : make_int2(0, p.W_R);
     float2 *T = Bt.T + ((size_t)z * p.wAa + i) * p.W_R;
 #pragma unroll
@@ -181,29 +230,27 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
             u[k] = (T + (size_t)(k * LM) * p.W_R)[at];
 #pragma unroll
         for (int k = 0; k < K; k++)
-            ldsf[(t % C) * G::PB + t / C + k * LM] = u[k];
+            G::region(ldsf, t % C)[t / C + k * LM] = u[k];
     }
     fftn::table<G::M>(tw);
     __syncthreads();
     if (t < C * LN) {
         const int j = t % LN;
-        const float2 *in = ldsf + (t / LN) * G::PB;
-        float2 *ex = ldsf + G::template at<LN>(t / LN);
+        float2 *io = G::region(ldsf, t / LN);
         float2 v[V];
 #pragma unroll
         for (int r = 0; r < V; r++)
-            v[r] = in[j + LN * r];
+            v[r] = io[j + LN * r];
         fft8::wave_sync();
-        fftn::fft<N, -1, G::M>(v, j, ex, tw);
+        fftn::fft<N, -1, G::M>(v, j, G::template ex<LN>(ldsf, t / LN), tw);
 #pragma unroll
         for (int r = 0; r < V; r++)
-            ex[j + LN * r] = v[r];
+            io[j + LN * r] = v[r];
     }
     __syncthreads();
     {
         const int j = t % LM, az = Bt.az[b];
-        const float2 *in = ldsf + G::template at<LN>(t / LM);
-        float2 *ex = ldsf + G::template at<LM>(t / LM);
+        const float2 *in = G::region(ldsf, t / LM);
         float2 v[V];
 #pragma unroll
         for (int r = 0; r < V; r++) {
@@ -215,8 +262,8 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
             }
         }
         fft8::wave_sync();
-        fftn::fft<M, +1, G::M>(v, j, ex, tw);
-        float *exf = (float *)(ldsf + (t / LM) * G::PB);
+        fftn::fft<M, +1, G::M>(v, j, G::template ex<LM>(ldsf, t / LM), tw);
+        float *exf = (float *)G::region(ldsf, t / LM);
 #pragma unroll
         for (int r = 0; r < V; r++) {
 #pragma clang fp contract(off)
@@ -228,7 +275,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_cols(WPar p, WBatch Bt, 
     const unsigned at = (t / C) * p.W_R + t % C;
 #pragma unroll
     for (int k = 0; k < M / LM; k++)
-        (U + (size_t)(k * LM) * p.W_R)[at] = ((const float *)(ldsf + (t % C) * G::PB))[t / C + k * LM];
+        (U + (size_t)(k * LM) * p.W_R)[at] = ((const float *)G::region(ldsf, t % C))[t / C + k * LM];
 }
 
 template <int N>
@@ -251,7 +298,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_zrows(WPar p, WBatch Bt,
     }
     fftn::table<G::M>(tw);
     __syncthreads();
-    fftn::fft<G::M, -1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
+    fftn::fft<G::M, -1, G::M>(v, j, G::template ex<LM>(ldsf, t / LM), tw);
     float2 *Z = Bt.Zs + ((size_t)b * p.W_A + y) * p.W_R + j;
 #pragma unroll
     for (int r = 0; r < V; r++)
@@ -259,7 +306,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_zrows(WPar p, WBatch Bt,
 }
 
 template <int N>
-__global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_urows(WPar p, WfBatch F)
+__global__ void __launch_bounds__(WfGeom<N>::NTHR, 4) k_wf_urows(WPar p, WfBatch F)
 {
     using G = WfGeom<N>;
     constexpr int V = G::VM, M = G::M, LM = G::LM;
@@ -273,7 +320,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHR) k_wf_urows(WPar p, WfBatch F)
         v[r] = Gq[LM * r];
     fftn::table<G::M>(tw);
     __syncthreads();
-    fftn::fft<M, +1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
+    fftn::fft<M, +1, G::M>(v, j, G::template ex<LM>(ldsf, t / LM), tw);
     const int lagR = WOS * p.epR;
     float2 *X = F.X + ((size_t)q * p.W_A + y) * F.pitchX;
 #pragma unroll
@@ -315,7 +362,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC) k_wf_lags(WPar p, WfBatch F, 
     for (int r = 0; r < V; r++)
         v[r] = ex[j + LM * r];
     fft8::wave_sync();
-    fftn::fft<M, +1, G::M>(v, j, ldsf + G::template at<LM>(t / LM), tw);
+    fftn::fft<M, +1, G::M>(v, j, G::template full<LM>(ldsf, t / LM), tw);
     fft8::wave_sync();
 #pragma unroll
     for (int r = 0; r < V; r++)
@@ -506,7 +553,7 @@ __global__ void __launch_bounds__(WfGeom<N>::NTHC, 2) k_wf_cross(WPar p, WBatch 
     const int Lb = flat < per * 8 ? (flat % 8) * per + flat / 8 : flat;
     const int q = Lb / nbx, c0 = (Lb - q * nbx) * C, t = threadIdx.x, W = p.W_R, H = W / 2;
     const int j = t % LM, slot = t / LM;
-    float2 *ex = ldsf + slot * G::PB, *sx = ldsf + G::template at<LM>(slot);
+    float2 *ex = ldsf + slot * G::PB, *sx = G::template full<LM>(ldsf, slot);
     const bool self = c0 + slot == 0;
     fftn::table<G::M>(tw);
     // column of load / store lane t % C on side s (0: l, 1: mirror)
