@@ -50,14 +50,12 @@ struct AmpGeom {
 __device__ inline void amp_detect(const float2 (&y)[8], float scale, float (&x)[8], float (&a)[8])
 {
     constexpr int H = 8;
-    bool tiny = false;
 #pragma unroll
     for (int j = 0; j < H; j++) {
 #pragma clang fp contract(off)
         x[j] = (y[j].x * y[j].x + y[j].y * y[j].y) * scale;
-        tiny |= !(x[j] >= 0x1p-96f);
     }
-    if (__builtin_amdgcn_ballot_w64(tiny) == 0) {
+    if (!sqrt_needs_full(x)) {
 #pragma unroll
         for (int j = 0; j < H; j++)
             a[j] = sqrt_rn_normal(x[j]);

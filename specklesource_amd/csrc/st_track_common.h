@@ -398,16 +398,37 @@ __device__ inline void refine_fine(unsigned char *scr, int t, Sync sync, double 
 #pragma clang fp contract(off)
 // 1-D Gaussian LM fit (gaussPeak1D / mrqminMod / mrqcofMod / myGauss1D,
 // speckleTrack.c:2137-2202, 2309-2465), all in float like the reference.
-__device__ inline void lm_gauss(float x, const float a[3], float *y, float dyda[3])
+//
+// Bound: FP64 and FP32 issue and, in small runs, latency: a serial chain of at
+// most six passes over 18 samples.  The divisors are the fit's, not the
+// sample's, so two FP64 reciprocals per pass replace three divisions per
+// sample: a quotient of two floats is the float rounding of the product with
+// the divisor's reciprocal (it is never within 2^-49 of a rounding boundary,
+// nor on one), the exponent's FP64 quotient takes the rounded product and its
+// exact residual; both are the correctly rounded ones.
+
+// exp(-t), t >= 0 or NaN, to 2^-50 (the caller rounds it to float): t log2(e)
+// split into a whole number and a rest, Taylor's series of the rest (|r| <=
+// ln 2 / 2, terms to r^12, even and odd ones in two chains).
+__device__ inline double lm_exp_neg(double t)
 {
-    float sig = a[2];
-    float t = x - a[1];
-    float argx = (float)(0.5 * (double)t * (double)t / (double)(sig * sig));
-    float ex = (float)exp(-(double)argx);
-    *y = a[0] * ex;
-    dyda[0] = ex;
-    dyda[1] = *y * t / (sig * sig);
-    dyda[2] = *y * t * t / (sig * sig * sig);
+    t = t > 800.0 ? 800.0 : t;  // far below every float
+    const double n = __builtin_rint(t * -1.4426950408889634);
+    // ln 2 in 32 bits and the rest
+    const double r = fma(-n, -4.2009150726810846e-11, fma(-n, 0.6931471806019545, -t)), q = r * r;
+    double e = 1.0 / 479001600, o = 1.0 / 39916800;
+    e = fma(e, q, 1.0 / 3628800);
+    o = fma(o, q, 1.0 / 362880);
+    e = fma(e, q, 1.0 / 40320);
+    o = fma(o, q, 1.0 / 5040);
+    e = fma(e, q, 1.0 / 720);
+    o = fma(o, q, 1.0 / 120);
+    e = fma(e, q, 1.0 / 24);
+    o = fma(o, q, 1.0 / 6);
+    e = fma(e, q, 0.5);
+    o = fma(o, q, 1.0);
+    e = fma(e, q, 1.0);
+    return __builtin_amdgcn_ldexp(fma(o, r, e), (int)n);
 }
 
 __device__ inline void lm_coef(const float *x, const float *y, const float a[3], float alpha[3][3], float beta[3],
@@ -421,9 +442,18 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
     *chisq = 0.0f;
     const float sg = 0.1f;
     const float sig2i = (float)(1.0 / (double)(sg * sg));
+    const float s2 = a[2] * a[2], s3 = s2 * a[2];
+    const double d2 = (double)s2, r2 = 1.0 / d2, r3 = 1.0 / (double)s3;
+    const bool residual = s2 > 1e-30f && s2 < 1e30f;  // zero, infinite, NaN: the division itself
     for (int i = 0; i < NGAUSS; i++) {
-        float ymod, dyda[3];
-        lm_gauss(x[i], a, &ymod, dyda);
+        // myGauss1D
+        const float t = x[i] - a[1];
+        const double num = 0.5 * (double)t * (double)t;
+        double arg = num * r2;
+        arg = residual ? fma(fma(-arg, d2, num), r2, arg) : num / d2;
+        const float ex = (float)lm_exp_neg((double)(float)arg);
+        const float ymod = a[0] * ex;
+        const float dyda[3] = {ex, (float)((double)(ymod * t) * r2), (float)((double)(ymod * t * t) * r3)};
         float dy = y[i] - ymod;
         for (int l = 0; l < 3; l++) {
             float wt = dyda[l] * sig2i;
@@ -498,8 +528,9 @@ __device__ inline float gauss_peak_1d(const float *yin, float x0)
         y[i] = yin[i];
         maxC = y[i] > maxC ? y[i] : maxC;
     }
+    const double rmax = 1.0 / (double)maxC;
     for (int i = 0; i < NGAUSS; i++)
-        y[i] /= maxC;
+        y[i] = (float)((double)y[i] * rmax);  // y / maxC
     float a[3] = {1.0f, x[NGAUSS / 2], 2.0f};
     float alpha[3][3], beta[3], ochisq, chisq;
     float lambda = 0.001f;
