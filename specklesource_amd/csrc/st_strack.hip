@@ -2389,6 +2389,12 @@ __global__ void __launch_bounds__(2 * FusedLanes<W>::L * W) __attribute__((amdgp
     __shared__ int stz[NTH / 64], sflag[2];
     __shared__ unsigned smask[NTH];
     __shared__ int srank;  // rank of the surface maximum (atomicMin over its holders)
+    // exp(i pi s / w), s the signed frequency of index rho.  From LDS: selected
+    // per lane half from scalar constants it cost nine instructions per element
+    // (64 px scene 7869 -> 7400 us).
+    __shared__ __align__(16) float2 rot[W];
+    if (threadIdx.x < W)
+        rot[threadIdx.x] = c_tw128[((threadIdx.x < W / 2 ? threadIdx.x : threadIdx.x - W) * (64 / W)) & 127];
     constexpr bool isf = STYPE == ST_SAMPLE_C64;
     const float thr = isf ? 1e-15f : 1e-9f;
 
@@ -2567,11 +2573,13 @@ __global__ void __launch_bounds__(2 * FusedLanes<W>::L * W) __attribute__((amdgp
         // ---------------- cross spectrum X = F1 conj(F2), row r, half h
         {
             const float2 *Fo = lds + (size_t)(1 - g) * BUF;
+            const float sg = g ? -1.f : 1.f;
 #pragma unroll
             for (int k = 0; k < H; k++) {
 #pragma clang fp contract(off)
-                const float2 o = Fo[FL::at(r, blk * H + k)];
-                x[k] = g == 0 ? cmulconj(x[k], o) : cmulconj(o, x[k]);
+                // group 1 forms F2 conj(F1), the conjugate
+                const float2 o = Fo[FL::at(r, blk * H + k)], c = cmulconj(x[k], o);
+                x[k] = make_float2(c.x, sg * c.y);
             }
         }
         __syncthreads();
@@ -2591,15 +2599,7 @@ __global__ void __launch_bounds__(2 * FusedLanes<W>::L * W) __attribute__((amdgp
 #pragma unroll
             for (int k = 0; k < H; k++) {
                 // column l = blk H + k, signed frequency (Nyquist negative)
-                float2 cf = c_tw128[(k * (64 / W)) & 127];
-#pragma unroll
-                for (int b2 = 1; b2 < L; b2++) {
-                    const int l = b2 * H + k;
-                    const int ls = l < W / 2 ? l : l - W;
-                    const float2 cb = c_tw128[(ls * (64 / W)) & 127];
-                    cf = blk == b2 ? cb : cf;
-                }
-                x[k] = cmul_f(x[k], cf);
+                x[k] = cmul_f(x[k], rot[blk * H + k]);
             }
         }
         LF::inv(x, h);
@@ -2648,15 +2648,7 @@ __global__ void __launch_bounds__(2 * FusedLanes<W>::L * W) __attribute__((amdgp
 #pragma unroll
             for (int k = 0; k < H; k++) {
                 // row blk H + k, signed frequency k - blk H (L = 2)
-                float2 rf = c_tw128[(k * (64 / W)) & 127];
-#pragma unroll
-                for (int b2 = 1; b2 < L; b2++) {
-                    const int rho = b2 * H + k;
-                    const int rs = rho < W / 2 ? rho : rho - W;
-                    const float2 cb = c_tw128[(rs * (64 / W)) & 127];
-                    rf = blk == b2 ? cb : rf;
-                }
-                y[k] = cmul_f(Z[FL::at(blk * H + k, r)], rf);
+                y[k] = cmul_f(Z[FL::at(blk * H + k, r)], rot[blk * H + k]);
             }
             __syncthreads();  // every read of Z done: the LDS takes the surface
             LF::inv(y, h);
@@ -2748,13 +2740,6 @@ __global__ void __launch_bounds__(2 * FusedLanes<W>::L * W) __attribute__((amdgp
 constexpr int kF128 = 128;
 constexpr size_t kF128SlotM = (size_t)4 * kF128 * kF128;  // float per workgroup: |C|
 
-// exp(i pi (blk 32 + k - (blk >= 2 ? 128 : 0)) / 128) = s_blk exp(i pi k / 128):
-// the polyphase factor of the signed frequency of element k of block blk
-__device__ inline float2 f128_factor(float2 sblk, int k)
-{
-    return ::fftreg::cmul_f(sblk, make_float2(::fftreg::kTw256Re[k], ::fftreg::kTw256Im[k]));
-}
-
 template <int STYPE>
 __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ Pp, const Pts *__restrict__ Sp,
                                                       const int *__restrict__ jobStart, int njobs,
@@ -2763,6 +2748,12 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
     constexpr int W = kF128, L = 4, H = W / L, NTH = 512, WW = 2 * W;
     using FL = FusedLanes<W>;
     extern __shared__ float2 lds[];  // [BUF]: the transpose buffer
+    // exp(i pi s / 128), s the signed frequency of index rho: the polyphase factors
+    __shared__ __align__(16) float2 rot[W];
+    if (threadIdx.x < W) {
+        const float2 c = fft8::c_tw256[(threadIdx.x < W / 2 ? threadIdx.x : threadIdx.x - W) & 255];
+        rot[threadIdx.x] = make_float2(c.x, -c.y);
+    }
     __shared__ Top2 sht[NTH / 64];
     constexpr bool isf = STYPE == ST_SAMPLE_C64;
     const int count = jobStart[njobs];
@@ -2868,12 +2859,6 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
         }
         // ---------------- polyphase inverse, one column phase q at a time
         const int krow = ((r - az) % W + W) % W;
-        // s_blk = exp(i pi (blk 32 - (blk >= 2 ? 128 : 0)) / 128): 1, exp(i pi / 4), -i, -exp(i 3 pi / 4)
-        auto sblk_of = [](int b) {
-            const float c45 = 0x1.6a09e6p-1f;
-            return b == 0 ? make_float2(1.f, 0.f)
-                   : b == 1 ? make_float2(c45, c45) : b == 2 ? make_float2(0.f, -1.f) : make_float2(c45, -c45);
-        };
         const int Jq = (2 * r + W) & (WW - 1);  // surface column of q = 0 (q = 1: + 1)
         Top2 best{0.0f, 0x7fffffff, 0.0f, 0.0f};
 #pragma unroll 1
@@ -2882,11 +2867,10 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
                 int h = t & 3;
                 asm volatile("" : "+v"(h));
                 const int blk = ::fftreg::qblk(h);
-                const float2 sblk = sblk_of(blk);
                 float2 x[H];
 #pragma unroll
                 for (int k = 0; k < H; k++)  // column l = blk 32 + k: exp(i pi ls / 128) on phase 1
-                    x[k] = q ? ::fftreg::cmul_f(Xr[k], f128_factor(sblk, k)) : Xr[k];
+                    x[k] = q ? ::fftreg::cmul_f(Xr[k], rot[blk * H + k]) : Xr[k];
                 ::fftreg::inv_quad128(x, h);  // x[n'] = Z[krow][L n' + h]
 #pragma unroll
                 for (int n = 0; n < H; n++)
@@ -2899,13 +2883,12 @@ __global__ void __launch_bounds__(512) k_cpx_fused128(const KPar *__restrict__ P
                 int h = t & 3;
                 asm volatile("" : "+v"(h));
                 const int blk = ::fftreg::qblk(h);
-                const float2 sblk = sblk_of(blk);
                 float2 y[H];
 #pragma unroll
                 for (int k = 0; k < H; k++) {
                     y[k] = lds[FL::at(blk * H + k, r)];
                     if (pp)  // row rho = blk 32 + k: exp(i pi rs / 128)
-                        y[k] = ::fftreg::cmul_f(y[k], f128_factor(sblk, k));
+                        y[k] = ::fftreg::cmul_f(y[k], rot[blk * H + k]);
                 }
                 ::fftreg::inv_quad128(y, h);  // y[j] = C_pp,q[L j + h][r]
                 // |C|^2 first; a wave with no value below 2^-96 (nearly always)
