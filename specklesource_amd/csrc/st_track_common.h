@@ -444,13 +444,14 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
     const float sig2i = (float)(1.0 / (double)(sg * sg));
     const float s2 = a[2] * a[2], s3 = s2 * a[2];
     const double d2 = (double)s2, r2 = 1.0 / d2, r3 = 1.0 / (double)s3;
-    const bool residual = s2 > 1e-30f && s2 < 1e30f;  // zero, infinite, NaN: the division itself
+    const bool finite = s2 > 0.0f && s2 <= 3.402823466e38f;  // else the product is the quotient, or NaN as it is
     for (int i = 0; i < NGAUSS; i++) {
         // myGauss1D
         const float t = x[i] - a[1];
         const double num = 0.5 * (double)t * (double)t;
         double arg = num * r2;
-        arg = residual ? fma(fma(-arg, d2, num), r2, arg) : num / d2;
+        const double whole = fma(fma(-arg, d2, num), r2, arg);
+        arg = finite ? whole : arg;
         const float ex = (float)lm_exp_neg((double)(float)arg);
         const float ymod = a[0] * ex;
         const float dyda[3] = {ex, (float)((double)(ymod * t) * r2), (float)((double)(ymod * t * t) * r3)};
@@ -468,51 +469,73 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
             alpha[k][j] = alpha[j][k];
 }
 
-// Gauss-Jordan with full pivoting on a 3x3 system; 0 when singular.
+// Gauss-Jordan with full pivoting on a 3x3 system; 0 when singular.  Rows are
+// swapped so that a pivot stands on the diagonal, so b ends in order; the
+// columns of spent pivots, which b does not depend on, are left behind.  Every
+// element has a fixed register: the pivot search carries indices along, swaps
+// are selects, the elimination is one of three (with indices into the arrays,
+// element selects were half of the whole fit).
+template <int C>
+__device__ inline void solve3_eliminate(float m[3][3], float b[3], float pinv)
+{
+    for (int l = 0; l < 3; l++)
+        if (l != C)
+            m[C][l] *= pinv;
+    b[C] *= pinv;
+    for (int ll = 0; ll < 3; ll++)
+        if (ll != C) {
+            const float d = m[ll][C];
+            for (int l = 0; l < 3; l++)
+                if (l != C)
+                    m[ll][l] -= m[C][l] * d;
+            b[ll] -= b[C] * d;
+        }
+}
+
 __device__ inline int solve3(float m[3][3], float b[3])
 {
-    int used[3] = {0, 0, 0};
+    unsigned used = 0;
+#pragma unroll
     for (int it = 0; it < 3; it++) {
         float big = 0;
         int r = -1, c = -1;
-        for (int j = 0; j < 3; j++) {
-            if (used[j])
-                continue;
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+#pragma unroll
             for (int k = 0; k < 3; k++)
-                if (!used[k] && fabsf(m[j][k]) >= big) {
+                if (!(used >> j & 1) && !(used >> k & 1) && fabsf(m[j][k]) >= big) {
                     big = fabsf(m[j][k]);
                     r = j;
                     c = k;
                 }
-        }
         if (r < 0)
             return 0;
-        used[c] = 1;
-        if (r != c) {
-            for (int l = 0; l < 3; l++) {
-                float t = m[r][l];
-                m[r][l] = m[c][l];
-                m[c][l] = t;
+        used |= 1u << c;
+#pragma unroll
+        for (int lo = 0; lo < 2; lo++)
+#pragma unroll
+            for (int hi = lo + 1; hi < 3; hi++) {
+                const bool swap = r != c && min(r, c) == lo && max(r, c) == hi;
+#pragma unroll
+                for (int l = 0; l < 3; l++) {
+                    const float x = m[lo][l], y = m[hi][l];
+                    m[lo][l] = swap ? y : x;
+                    m[hi][l] = swap ? x : y;
+                }
+                const float x = b[lo], y = b[hi];
+                b[lo] = swap ? y : x;
+                b[hi] = swap ? x : y;
             }
-            float t = b[r];
-            b[r] = b[c];
-            b[c] = t;
-        }
-        if (m[c][c] == 0.0f)
+        const float pivot = c == 0 ? m[0][0] : c == 1 ? m[1][1] : m[2][2];
+        if (pivot == 0.0f)
             return 0;
-        float pinv = (float)(1.0 / (double)m[c][c]);
-        m[c][c] = 1.0f;
-        for (int l = 0; l < 3; l++)
-            m[c][l] *= pinv;
-        b[c] *= pinv;
-        for (int ll = 0; ll < 3; ll++)
-            if (ll != c) {
-                float d = m[ll][c];
-                m[ll][c] = 0.0f;
-                for (int l = 0; l < 3; l++)
-                    m[ll][l] -= m[c][l] * d;
-                b[ll] -= b[c] * d;
-            }
+        const float pinv = (float)(1.0 / (double)pivot);
+        if (c == 0)
+            solve3_eliminate<0>(m, b, pinv);
+        else if (c == 1)
+            solve3_eliminate<1>(m, b, pinv);
+        else
+            solve3_eliminate<2>(m, b, pinv);
     }
     return 1;
 }
