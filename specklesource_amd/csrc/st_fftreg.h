@@ -46,30 +46,6 @@ constexpr int bitrev(int i)
     return j;
 }
 
-// Butterfly a + w b, a - w b with w = exp(SIGN 2 pi i k / len) in six FMAs
-// (the multiplication split as c (1, s / c), or s (c / s, 1) where |s| > |c|,
-// so both outputs take the common factor inside their own FMA): two
-// roundings per output component instead of three, six instructions instead
-// of eight.
-template <int SIGN>
-__device__ inline void bfly(float2 &a, float2 &b, int k, int len)
-{
-    const float2 w = tw<SIGN>(k, len);
-    float2 u;
-    float f;
-    if (__builtin_fabsf(w.x) >= __builtin_fabsf(w.y)) {
-        const float r = (float)((double)w.y / (double)w.x);
-        u = make_float2(fmaf(-r, b.y, b.x), fmaf(r, b.x, b.y));
-        f = w.x;
-    } else {
-        const float r = (float)((double)w.x / (double)w.y);
-        u = make_float2(fmaf(r, b.x, -b.y), fmaf(r, b.y, b.x));
-        f = w.y;
-    }
-    b = make_float2(fmaf(-f, u.x, a.x), fmaf(-f, u.y, a.y));
-    a = make_float2(fmaf(f, u.x, a.x), fmaf(f, u.y, a.y));
-}
-
 // In-place N-point FFT, natural order in and out.
 template <int N, int SIGN>
 __device__ inline void fft(float2 (&x)[N])
@@ -89,12 +65,14 @@ __device__ inline void fft(float2 (&x)[N])
         for (int i = 0; i < N; i += len) {
 #pragma unroll
             for (int k = 0; k < len / 2; k++) {
-                if (k != 0 && 4 * k != len) {
-                    bfly<SIGN>(x[i + k], x[i + k + len / 2], k, len);
-                    continue;
-                }
                 const float2 a = x[i + k], b = x[i + k + len / 2];
-                const float2 tb = k == 0 ? b : (SIGN < 0 ? make_float2(b.y, -b.x) : make_float2(-b.y, b.x));
+                float2 tb;
+                if (k == 0)
+                    tb = b;
+                else if (4 * k == len)
+                    tb = SIGN < 0 ? make_float2(b.y, -b.x) : make_float2(-b.y, b.x);
+                else
+                    tb = cmul_f(b, tw<SIGN>(k, len));
                 x[i + k] = make_float2(a.x + tb.x, a.y + tb.y);
                 x[i + k + len / 2] = make_float2(a.x - tb.x, a.y - tb.y);
             }
@@ -142,25 +120,26 @@ __device__ inline void fwd_pair(float2 (&x)[W / 2], int h)
 }
 
 // Inverse (exp(+2 pi i jk/W)) W-point FFT over a lane pair.  Lane h holds
-// inputs h*W/2 + n; on return it holds outputs 2k + h.  Lane 0 takes the
-// sum, lane 1 the difference (one sign-selected FMA) times the twiddle; the
-// product is formed on both and selected, so every twiddle stays a literal
-// (a lane-selected twiddle held 72 registers too many at W = 64).
+// inputs h*W/2 + n; on return it holds outputs 2k + h.  (Forming the
+// butterfly as in fwd_pair, one sign-selected add and a per-lane twiddle,
+// raised register pressure here: 72 VGPRs spilled at W = 64.)
 template <int W>
 __device__ inline void inv_pair(float2 (&x)[W / 2], int h)
 {
     constexpr int H = W / 2;
-    const float sg = h ? -1.f : 1.f;
 #pragma unroll
     for (int n = 0; n < H; n++) {
         const float2 y = shfl_pair(x[n]);
-        const float2 d = make_float2(fmaf(sg, x[n].x, y.x), fmaf(sg, x[n].y, y.y));
+        const float2 a = make_float2(x[n].x + y.x, x[n].y + y.y);
+        const float2 d = make_float2(y.x - x[n].x, y.y - x[n].y);
+        float2 b;
         if (n == 0)
-            x[n] = d;
-        else {
-            const float2 b = 4 * n == W ? make_float2(-d.y, d.x) : cmul_f(d, tw<+1>(n, W));
-            x[n] = h ? b : d;
-        }
+            b = d;
+        else if (4 * n == W)
+            b = make_float2(-d.y, d.x);
+        else
+            b = cmul_f(d, tw<+1>(n, W));
+        x[n] = h ? b : a;
     }
     fft<H, +1>(x);
 }
@@ -214,7 +193,6 @@ __device__ inline float2 twx(int k, int len)
 template <int XOR, int SIGN, int LEN>
 __device__ inline void quad_fwd_stage(float2 (&x)[32], int role, int rot)
 {
-    const float sg = role ? -1.f : 1.f;
 #pragma unroll
     for (int k = 0; k < 32; k++) {
         float2 m = cmul_f(x[k], twx<SIGN>(k, LEN));
@@ -222,7 +200,7 @@ __device__ inline void quad_fwd_stage(float2 (&x)[32], int role, int rot)
             m = SIGN < 0 ? make_float2(m.y, -m.x) : make_float2(-m.y, m.x);
         const float2 t = role ? m : x[k];
         const float2 y = shfl_quad<XOR>(t);
-        x[k] = make_float2(fmaf(sg, t.x, y.x), fmaf(sg, t.y, y.y));
+        x[k] = role ? make_float2(y.x - t.x, y.y - t.y) : make_float2(y.x + t.x, y.y + t.y);
     }
 }
 
@@ -232,15 +210,15 @@ __device__ inline void quad_fwd_stage(float2 (&x)[32], int role, int rot)
 template <int XOR, int SIGN, int LEN>
 __device__ inline void quad_inv_stage(float2 (&x)[32], int role, int rot)
 {
-    const float sg = role ? -1.f : 1.f;
 #pragma unroll
     for (int n = 0; n < 32; n++) {
         const float2 y = shfl_quad<XOR>(x[n]);
-        const float2 d = make_float2(fmaf(sg, x[n].x, y.x), fmaf(sg, x[n].y, y.y));
+        const float2 a = make_float2(x[n].x + y.x, x[n].y + y.y);
+        const float2 d = make_float2(y.x - x[n].x, y.y - x[n].y);
         float2 m = cmul_f(d, twx<SIGN>(n, LEN));
         if (rot)
             m = SIGN < 0 ? make_float2(m.y, -m.x) : make_float2(-m.y, m.x);
-        x[n] = role ? m : d;
+        x[n] = role ? m : a;
     }
 }
 
