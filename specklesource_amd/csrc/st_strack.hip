@@ -426,15 +426,39 @@ __global__ void __launch_bounds__(kIntThreads) k_int_bins_g(KPar P, Pts S, const
     }
 }
 
+// Counters and list slots by the workgroup: one atomic for kCountThreads points
+// (all of them call; the caller's slot, if it takes one).  Atomics of all waves
+// to one address run one after the other, some 10 ns each from eight dies.
+// 179 k points, one per wave -> here: k_cpx_finalize 71 -> 20, k_geometry 38 -> 11 us.
+constexpr int kCountThreads = 512;
+__device__ inline int block_count(int *counter, bool take)
+{
+    __shared__ int sw[kCountThreads / 64], base;
+    const unsigned long long m = __ballot(take);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (lane == 0)
+        sw[wid] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int w = 0; w < kCountThreads / 64; w++)
+            n += sw[w];
+        base = n ? atomicAdd(counter, n) : 0;
+    }
+    __syncthreads();
+    int k = base + __popcll(m & ((1ull << lane) - 1));
+    for (int w = 0; w < wid; w++)
+        k += sw[w];
+    __syncthreads();  // the next call's writes come after these reads
+    return k;
+}
+
 // ---------------------------------------------------------------------
 // geometry: findImage2Pos (polynomial) or host-computed positions,
 // maskValue, complex eligibility; initialises the point state.
-__global__ void k_geometry(KPar P, Pts S, const int *hostR2, const int *hostA2, int *list)
+__device__ inline bool geometry_point(const KPar &P, const Pts &S, const int *hostR2, const int *hostA2, int pt)
 {
     const int npts = P.nR * P.nA;
-    const int pt = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pt >= npts)
-        return;
     const int i = pt / P.nR, j = pt - i * P.nR;
     const int a1 = P.aStart + i * P.deltaA - P.wA / 2;
     const int r1 = P.rStart + j * P.deltaR - P.wR / 2;
@@ -484,10 +508,17 @@ __global__ void k_geometry(KPar P, Pts S, const int *hostR2, const int *hostA2, 
         S.sigRg[o] = S.sigAz[o] = S.peakGap[o] = S.fineGap[o] = S.snr[o] = 0.f;
     }
     const bool ok = in_bounds(r1, a1, P.wR, P.wA, P.im.nr1, P.im.na1) && in_bounds(r2, a2, P.wR, P.wA, P.im.nr2, P.im.na2);
-    if (ok && mv > 0 && !P.noComplex) {
-        int k = atomicAdd(&S.counts[CNT_LIST], 1);
+    return ok && mv > 0 && !P.noComplex;
+}
+
+__global__ void __launch_bounds__(kCountThreads) k_geometry(KPar P, Pts S, const int *hostR2, const int *hostA2,
+                                                            int *list)
+{
+    const int pt = blockIdx.x * kCountThreads + threadIdx.x;
+    const bool take = pt < P.nR * P.nA && geometry_point(P, S, hostR2, hostA2, pt);
+    const int k = block_count(&S.counts[CNT_LIST], take);
+    if (take)
         list[k] = pt;
-    }
 }
 
 // ---------------------------------------------------------------------
@@ -751,20 +782,16 @@ __global__ void __launch_bounds__(128) k_lm(const PeakRes *res, int B, float *si
 }
 
 // complexMatch tail + finalizeCmpxMatch (speckleTrack.c:377-394,714-739).
-__global__ void k_cpx_finalize(KPar P, Pts S, const int *list, int off, int B, CpxBatch C)
+// Bit 0: an attempt, bit 1: a match.
+__device__ inline int cpx_finalize_one(const KPar &P, const Pts &S, const int *list, int off, int b, const CpxBatch &C)
 {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B)
-        return;
     const int pt = list[off + b];
-    const int npts = P.nR * P.nA;
     if (!C.have[b]) {
         S.haveData[pt] = 0;
-        return;
+        return 0;
     }
     S.azValid[pt] = 1;
     S.azShift[pt] = C.az[b];
-    atomicAdd(&S.counts[CNT_CORR0], 1);
     const PeakRes &r = C.res[b];
     const double p1 = C.p[2 * b], p2 = C.p[2 * b + 1];
     double cMax;
@@ -799,7 +826,6 @@ __global__ void k_cpx_finalize(KPar P, Pts S, const int *list, int off, int B, C
                     good = 1;
                     S.rShift1[pt] = rs;
                     S.aShift1[pt] = as;
-                    atomicAdd(&S.counts[CNT_COMPLEX], 1);
                 }
             }
         }
@@ -820,7 +846,16 @@ __global__ void k_cpx_finalize(KPar P, Pts S, const int *list, int off, int B, C
     S.peakGap[pt] = r.gap;
     S.fineGap[pt] = r.fineGap;
     S.snr[pt] = r.snr;
-    (void)npts;
+    return good ? 3 : 1;
+}
+
+__global__ void __launch_bounds__(kCountThreads) k_cpx_finalize(KPar P, Pts S, const int *list, int off, int B,
+                                                                CpxBatch C)
+{
+    const int b = blockIdx.x * kCountThreads + threadIdx.x;
+    const int done = b < B ? cpx_finalize_one(P, S, list, off, b, C) : 0;
+    block_count(&S.counts[CNT_CORR0], done & 1);
+    block_count(&S.counts[CNT_COMPLEX], done & 2);
 }
 
 // Carry the last estimated azShift forward in raster order (the
@@ -897,15 +932,13 @@ __global__ void __launch_bounds__(kCarryBlk) k_carry_az(Pts S, int npts, const i
 }
 
 // Work list of the amplitude tries (the while loop of speckleTrack.c:246).
-__global__ void k_amp_list(KPar P, Pts S, int npts, int *list)
+__global__ void __launch_bounds__(kCountThreads) k_amp_list(KPar P, Pts S, int npts, int *list)
 {
-    const int pt = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pt >= npts)
-        return;
-    if (!S.good[pt] && S.haveData[pt] && S.maskv[pt] > 0) {
-        int k = atomicAdd(&S.counts[CNT_LIST], 1);
+    const int pt = blockIdx.x * kCountThreads + threadIdx.x;
+    const bool take = pt < npts && !S.good[pt] && S.haveData[pt] && S.maskv[pt] > 0;
+    const int k = block_count(&S.counts[CNT_LIST], take);
+    if (take)
         list[k] = pt;
-    }
 }
 
 // ---------------------------------------------------------------------
@@ -3704,7 +3737,7 @@ struct StrackJob {
             dA2 = upload(ctx, ha2.data(), ha2.size());
         }
         ST_HIP(hipMemsetAsync(S.counts, 0, CNT_N * sizeof(int), st));
-        hipLaunchKernelGGL(k_geometry, dim3((npts + 255) / 256), dim3(256), 0, st, P, S, dR2, dA2, list);
+        hipLaunchKernelGGL(k_geometry, dim3((npts + kCountThreads - 1) / kCountThreads), dim3(kCountThreads), 0, st, P, S, dR2, dA2, list);
         ST_HIP(hipGetLastError());
         ST_HIP(hipEventRecord(sev[1], st));
         nCpx = read_count(ctx, S.counts, CNT_LIST);
@@ -3773,7 +3806,8 @@ struct StrackJob {
                                nCpx, 2 * w, 0);
             ctx->time_end(kRef);
             hipLaunchKernelGGL(k_lm, dim3((2 * nCpx + 127) / 128), dim3(128), 0, st, C.res, nCpx, C.sig);
-            hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + 127) / 128), dim3(128), 0, st, P, S, list, 0, nCpx, C);
+            hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + kCountThreads - 1) / kCountThreads),
+                               dim3(kCountThreads), 0, st, P, S, list, 0, nCpx, C);
             ST_HIP(hipGetLastError());
             ar.used = mark;
         } else if (nCpx > 0 && !fusedPath) {
@@ -3833,7 +3867,8 @@ struct StrackJob {
                                        C.res, G);
                 ctx->time_end(kPeak);
                 hipLaunchKernelGGL(k_lm, dim3((2 * nb + 127) / 128), dim3(128), 0, st, C.res, nb, C.sig);
-                hipLaunchKernelGGL(k_cpx_finalize, dim3((nb + 127) / 128), dim3(128), 0, st, P, S, list, off, nb, C);
+                hipLaunchKernelGGL(k_cpx_finalize, dim3((nb + kCountThreads - 1) / kCountThreads),
+                               dim3(kCountThreads), 0, st, P, S, list, off, nb, C);
                 ST_HIP(hipGetLastError());
             }
             ar.used = mark;
@@ -3865,7 +3900,8 @@ struct StrackJob {
                            2 * w, 0);
         ctx->time_end(kRef);
         hipLaunchKernelGGL(k_lm, dim3((2 * nCpx + 127) / 128), dim3(128), 0, st, C.res, nCpx, C.sig);
-        hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + 127) / 128), dim3(128), 0, st, P, S, list, 0, nCpx, C);
+        hipLaunchKernelGGL(k_cpx_finalize, dim3((nCpx + kCountThreads - 1) / kCountThreads),
+                               dim3(kCountThreads), 0, st, P, S, list, 0, nCpx, C);
         ST_HIP(hipGetLastError());
     }
 
@@ -3946,7 +3982,7 @@ struct StrackJob {
         for (int t = 0; t < par.maxTries && t < 2; t++) {
             const int large = t;
             ST_HIP(hipMemsetAsync(S.counts + CNT_LIST, 0, sizeof(int), st));
-            hipLaunchKernelGGL(k_amp_list, dim3((npts + 255) / 256), dim3(256), 0, st, P, S, npts, list);
+            hipLaunchKernelGGL(k_amp_list, dim3((npts + kCountThreads - 1) / kCountThreads), dim3(kCountThreads), 0, st, P, S, npts, list);
             const int nA = read_count(ctx, S.counts, CNT_LIST);
             if (nA == 0)
                 break;
