@@ -133,23 +133,14 @@ __device__ inline void amp_no_match(const AmpBatch &A, int it, int st)
     A.res[it].I = A.res[it].J = -1000;
 }
 
-// Doppler shift of a window pair from lane_sums' totals, in units of ws, as
-// estDopCarrier1 and its rounding give it (patch_accept's expansion of the
-// lag sum around the mean).
+// Doppler shift of a window pair, in units of ws, from both windows' lag sums
+// (re, im), as estDopCarrier1 and its rounding give it: none for a sum that is
+// zero or not a number.
 template <int WS>
-__device__ inline int amp_doppler(const double (*s)[9])
+__device__ inline int amp_doppler(const double (*z)[2])
 {
-    const double cnt = (double)WS * (double)WS;
-    double zr[2], zi[2];
-    for (int g = 0; g < 2; g++) {
-        const double *T = s[g] + 1, *Lg = s[g] + 3, *F0 = s[g] + 5, *FL = s[g] + 7;
-        const double mr = T[0] / cnt, mi = T[1] / cnt;
-        const double s1r = T[0] - F0[0], s1i = T[1] - F0[1], s0r = T[0] - FL[0], s0i = T[1] - FL[1];
-        zr[g] = Lg[0] - (mr * s1r + mi * s1i) - (mr * s0r + mi * s0i) +
-                (double)(WS - 1) * (double)WS * (mr * mr + mi * mi);
-        zi[g] = Lg[1] - (mr * s1i - mi * s1r) - (mi * s0r - mr * s0i);
-    }
-    return doppler_round(zr[0], zi[0], zr[1], zi[1], WS, c_root256);
+    const double all = z[0][0] + z[0][1] + z[1][0] + z[1][1];  // finite samples give finite sums
+    return all == all ? doppler_round(z[0][0], z[0][1], z[1][0], z[1][1], WS, c_root256) : 0;
 }
 
 // The coarse peak of a try or its rejection near the border (findCPeak), and
@@ -199,12 +190,13 @@ k_amp_fused(KPar P, Pts S, const int *__restrict__ list, int count, int sc, AmpB
     constexpr int W = G::W, NTH = G::NTH, NW = NTH / 64, U = G::U, PB = G::PB;
     constexpr int LW = W / 8, LS = WS / 8;  // lanes per W-point and per ws-point transform
     constexpr int UH = U / 2;               // units per lane of the half-size passes
+    static_assert(UH == 1, "the Doppler sums of a window are complete after one turn");
     constexpr int SPAN = WS == 16 ? 32 : 64, NP = 2 * WS * LS / SPAN;  // partials of the Doppler sums, half per window
     constexpr bool isf = STYPE == ST_SAMPLE_C64;
     extern __shared__ float2 lds[];  // [W][PB]
     __shared__ AmpSums shs[NW], shp[NW];
     __shared__ Top2 sht[NW];
-    __shared__ double stp[NP][9];
+    __shared__ double stp[NP][4];  // Doppler partials: sums of the samples, of the lag products
     __shared__ int sAz, srank;
     const int Gr = gridDim.x, Q = Gr / 8;
     const int base = (Gr % 8 == 0) ? (blockIdx.x % 8) * Q + blockIdx.x / 8 : blockIdx.x;
@@ -249,33 +241,51 @@ k_amp_fused(KPar P, Pts S, const int *__restrict__ list, int count, int sc, AmpB
                 for (int r = 0; r < 8; r++)
                     v[r] = load(o + LS * r);
                 if constexpr (DOP != 0) {
-                    // Doppler sums of the row (PatchSums' order; [0] unused): the
-                    // window of a wave is one and the same (ws^2 / 8 units each)
-                    double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+                    // The mean first, then the lag products of what is left, as
+                    // doppler_shift does (one pass over the products with the mean
+                    // still in them loses the mean's share of the digits).  A wave's
+                    // units are of one window (ws^2 / 8 each).
+                    const bool lag = a > 0;
+                    const int e = u / SPAN;
+                    const bool last = (t & (SPAN - 1)) == SPAN - 1;
+                    float2 pv[8];
+#pragma unroll
+                    for (int r = 0; r < 8; r++)
+                        pv[r] = lag ? load(o - nr + LS * r) : make_float2(0.f, 0.f);
+                    double acc[2] = {0, 0};
 #pragma unroll
                     for (int r = 0; r < 8; r++) {
-                        const double vx = v[r].x, vy = v[r].y;
-                        acc[1] += vx;
-                        acc[2] += vy;
-                        if (a > 0) {
-                            const float2 pv = load(o - nr + LS * r);
-                            acc[3] = fma(vy, (double)pv.y, fma(vx, (double)pv.x, acc[3]));
-                            acc[4] = fma(-vx, (double)pv.y, fma(vy, (double)pv.x, acc[4]));
-                        }
-                    }
-                    if (a == 0) {
-                        acc[5] = acc[1];
-                        acc[6] = acc[2];
-                    }
-                    if (a == WS - 1) {
-                        acc[7] = acc[1];
-                        acc[8] = acc[2];
+                        acc[0] += v[r].x;
+                        acc[1] += v[r].y;
                     }
                     group_sum_last<SPAN>(acc);
-                    if ((t & (SPAN - 1)) == SPAN - 1)
+                    if (last) {
+                        stp[e][0] = acc[0];
+                        stp[e][1] = acc[1];
+                    }
+                    __syncthreads();
+                    double m[2] = {0, 0};
 #pragma unroll
-                        for (int k = 0; k < 9; k++)
-                            stp[u / SPAN][k] = acc[k];
+                    for (int k = 0; k < NP / 2; k++) {
+                        m[0] += stp[g * (NP / 2) + k][0];
+                        m[1] += stp[g * (NP / 2) + k][1];
+                    }
+                    constexpr double perSample = 1.0 / ((double)WS * WS);  // a power of two: exact
+                    m[0] *= perSample;
+                    m[1] *= perSample;
+                    acc[0] = acc[1] = 0;
+                    if (lag)
+#pragma unroll
+                        for (int r = 0; r < 8; r++) {
+                            const double ar = v[r].x - m[0], ai = v[r].y - m[1], br = pv[r].x - m[0], bi = pv[r].y - m[1];
+                            acc[0] += ar * br + ai * bi;
+                            acc[1] += ai * br - ar * bi;
+                        }
+                    group_sum_last<SPAN>(acc);
+                    if (last) {
+                        stp[e][2] = acc[0];
+                        stp[e][3] = acc[1];
+                    }
                 }
                 float2 *ex = row(a) + g * (WS + WS / 8);
                 fft8::fft<WS, -1>(v, j, ex, twS);
@@ -288,14 +298,11 @@ k_amp_fused(KPar P, Pts S, const int *__restrict__ list, int count, int sc, AmpB
         if (t == 0) {
             int az = S.azUse[w.pt];
             if constexpr (DOP != 0) {
-                double s[2][9];
-                for (int g = 0; g < 2; g++)
-                    for (int k = 0; k < 9; k++) {
-                        s[g][k] = stp[g * (NP / 2)][k];
-                        for (int e = 1; e < NP / 2; e++)
-                            s[g][k] += stp[g * (NP / 2) + e][k];
-                    }
-                az = (int)((float)amp_doppler<WS>(s) * (float)P.wA / (float)WS);
+                double z[2][2] = {{0, 0}, {0, 0}};
+                for (int e = 0; e < NP; e++)
+                    for (int k = 0; k < 2; k++)
+                        z[e / (NP / 2)][k] += stp[e][2 + k];
+                az = (int)((float)amp_doppler<WS>(z) * (float)P.wA / (float)WS);
                 S.azUse[w.pt] = az;
             }
             sAz = (int)((float)az * (float)WS / (float)P.wA);

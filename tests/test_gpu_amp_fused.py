@@ -57,6 +57,37 @@ def test_fused_tries_equal_staged_tries(device, monkeypatch, w, wa, stype):
         assert np.allclose(f.diag["snr"][t], s.diag["snr"][t], rtol=2e-5)
 
 
+@pytest.mark.parametrize("ulps", [0, 2])
+@pytest.mark.parametrize("wa", [16, 32, 64])
+def test_constant_windows(device, monkeypatch, wa, ulps):
+    """Float windows of one value each, and such windows with a noise of units
+    in the last place.  Of the former the lag sums after mean removal are zeros:
+    no Doppler shift, nothing to correlate.  Of the latter they are 2^-47 of the
+    windows' power, below the rounding of sums that keep the mean."""
+    T, n = wa + 4, 20
+    rng = np.random.default_rng(wa)
+
+    def tiles():
+        x = np.kron(rng.uniform(1, 2, (n, n, 2)).astype(np.float32), np.ones((T, T, 1), np.float32))
+        k = np.float32(2**-23) * rng.integers(-ulps, ulps + 1, x.shape)
+        return np.ascontiguousarray(x + k.astype(np.float32)).view(np.complex64)[..., 0]
+
+    p = small_params(wa, n * T, n * T, step=T, wRa=wa, wAa=wa, noComplex=1, rStart=T // 2, aStart=T // 2, nR=n, nA=n,
+                     maxTries=1)
+    pid = device.upload_pair(tiles(), tiles())
+    try:
+        f = device.speckle_track(pid, p, diag=True)
+        monkeypatch.setenv("SPECKLE_AMD_PATH", "staged")
+        s = device.speckle_track(pid, p, diag=True)
+    finally:
+        device.release_pair(pid)
+    assert ulps or (s.diag["peakI"][1] == -1000).all()
+    for k in ("offR", "offA", "azd", "type"):
+        assert np.array_equal(getattr(f, k), getattr(s, k)), k
+    for k in ("peakI", "peakJ", "fineI", "fineJ", "sigRg", "sigAz", "peakGap", "fineGap"):
+        assert np.array_equal(f.diag[k][1], s.diag[k][1]), k
+
+
 def test_one_try_and_no_try(device):
     """A single point, and a grid whose windows all leave the image."""
     a, b = _pair(160, 160, 3, abi.ST_SAMPLE_C64)
