@@ -1,0 +1,68 @@
+// Short forms of correctly rounded divisions and square roots
+// (tests/test_gpu_math.py compares them with the full ones).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace sttrack {
+
+// sqrtf for finite x >= 2^-96: the rounded product of x and its hardware
+// reciprocal square root, corrected by half its exact residual times the
+// latter.  Equal to sqrtf(x) at every such float (all 1.88e9 compared on
+// gfx950); five instructions against nine for the hardware root with its two
+// one-ulp tests, sixteen for sqrtf.
+__device__ inline float sqrt_rn_normal(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+}
+
+// Whether any of n values (sums of squares, so never negative) in the wave lies
+// outside sqrt_rn_normal's range, NaN included: least and greatest of the bit
+// patterns, two values an instruction.
+template <int n>
+__device__ inline bool sqrt_needs_full(const float (&x)[n])
+{
+    static_assert(n % 2 == 0, "pairs");
+    unsigned lo = 0xffffffffu, hi = 0;
+#pragma unroll
+    for (int j = 0; j < n; j += 2) {
+        const unsigned a = __float_as_uint(x[j]), b = __float_as_uint(x[j + 1]);
+        lo = min(lo, min(a, b));
+        hi = max(hi, max(a, b));
+    }
+    return __builtin_amdgcn_ballot_w64(lo < 0x0f800000u || hi >= 0x7f800000u) != 0;
+}
+
+// x / n, correctly rounded, from rn = 1 / n rounded (Markstein: the residual of
+// the rounded product is exact).  A product that is zero, infinite or NaN is
+// the quotient already, and its residual is not one.
+__device__ inline double div_by(double x, double n, double rn)
+{
+    constexpr int kFiniteNonzero = 0x198;  // classes: negative and positive, normal and subnormal
+    const double q = x * rn;
+    return __builtin_amdgcn_class(q, kFiniteNonzero) ? fma(fma(-q, n, x), rn, q) : q;
+}
+
+// x / sqrt(a).  Both from one reciprocal square root: coupled Newton steps
+// (Goldschmidt) give the root g and h = 1 / (2 g), a residual step rounds g,
+// another the quotient.  Zeros, negatives, subnormals, infinities and NaN take
+// the library's forms.
+__device__ inline double div_sqrt(double x, double a)
+{
+    if (!(a > 1e-280 && a < 1e280))
+        return x / sqrt(a);
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y, h = 0.5 * y;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const double e = fma(-h, g, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+    }
+    g = fma(fma(-g, g, a), h, g);
+    return div_by(x, g, h + h);
+}
+
+}  // namespace sttrack

@@ -25,6 +25,7 @@
 
 #include "st_ctx.h"
 #include "st_fftlds.h"
+#include "st_math.h"
 #include "st_track_common.h"
 #include "st_fftreg.h"
 #include "st_fft8.h"
@@ -1175,35 +1176,6 @@ __device__ inline Top2 wg_top2(Top2 a, Top2 *sh)
         __syncthreads();
         return r;
     }
-}
-
-// sqrtf for finite x >= 2^-96: the rounded product of x and its hardware
-// reciprocal square root, corrected by half its exact residual times the
-// latter.  Equal to sqrtf(x) at every such float (all 1.88e9 compared on
-// gfx950); five instructions against nine for the hardware root with its two
-// one-ulp tests, sixteen for sqrtf.
-__device__ inline float sqrt_rn_normal(float x)
-{
-    const float y = __builtin_amdgcn_rsqf(x);
-    const float s = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
-}
-
-// Whether any of n values (sums of squares, so never negative) in the wave lies
-// outside sqrt_rn_normal's range, NaN included: least and greatest of the bit
-// patterns, two values an instruction.
-template <int n>
-__device__ inline bool sqrt_needs_full(const float (&x)[n])
-{
-    static_assert(n % 2 == 0, "pairs");
-    unsigned lo = 0xffffffffu, hi = 0;
-#pragma unroll
-    for (int j = 0; j < n; j += 2) {
-        const unsigned a = __float_as_uint(x[j]), b = __float_as_uint(x[j + 1]);
-        lo = min(lo, min(a, b));
-        hi = max(hi, max(a, b));
-    }
-    return __builtin_amdgcn_ballot_w64(lo < 0x0f800000u || hi >= 0x7f800000u) != 0;
 }
 
 // The peak scan without ranks: each thread keeps the largest value, the

@@ -27,6 +27,7 @@
 #include "st_ctx.h"
 #include "st_fftlds.h"
 #include "st_fftn.h"
+#include "st_math.h"
 #include "st_track_common.h"
 
 using namespace sttrack;
@@ -510,34 +511,6 @@ __device__ inline void wave_scan(double (&x)[n])
     step(integral_constant<int, 0x118>(), integral_constant<int, 0xf>());
     step(integral_constant<int, 0x142>(), integral_constant<int, 0xa>());
     step(integral_constant<int, 0x143>(), integral_constant<int, 0xc>());
-}
-
-// x / n, correctly rounded, from rn = 1 / n rounded (Markstein: the residual of
-// the rounded product is exact).
-__device__ inline double div_by(double x, double n, double rn)
-{
-    const double q = x * rn;
-    return fma(fma(-q, n, x), rn, q);
-}
-
-// x / sqrt(a).  Both from one reciprocal square root: coupled Newton steps
-// (Goldschmidt) give the root g and h = 1 / (2 g), a residual step rounds g,
-// another the quotient.  Zeros, negatives, subnormals, infinities and NaN take
-// the library's forms.
-__device__ inline double div_sqrt(double x, double a)
-{
-    if (!(a > 1e-280 && a < 1e280))
-        return x / sqrt(a);
-    const double y = __builtin_amdgcn_rsq(a);
-    double g = a * y, h = 0.5 * y;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const double e = fma(-h, g, 0.5);
-        g = fma(g, e, g);
-        h = fma(h, e, h);
-    }
-    g = fma(fma(-g, g, a), h, g);
-    return div_by(x, g, h + h);
 }
 
 // computeMeanSigma (corrTrackFast.c:407-477, search part) and getPeakCorr
