@@ -35,20 +35,23 @@ __device__ inline bool sqrt_needs_full(const float (&x)[n])
     return __builtin_amdgcn_ballot_w64(lo < 0x0f800000u || hi >= 0x7f800000u) != 0;
 }
 
+constexpr int kFiniteNonzero = 0x198;  // classes: negative and positive, normal and subnormal
+
 // x / n, correctly rounded, from rn = 1 / n rounded (Markstein: the residual of
 // the rounded product is exact).  A product that is zero, infinite or NaN is
 // the quotient already, and its residual is not one.
 __device__ inline double div_by(double x, double n, double rn)
 {
-    constexpr int kFiniteNonzero = 0x198;  // classes: negative and positive, normal and subnormal
     const double q = x * rn;
     return __builtin_amdgcn_class(q, kFiniteNonzero) ? fma(fma(-q, n, x), rn, q) : q;
 }
 
-// x / sqrt(a).  Both from one reciprocal square root: coupled Newton steps
-// (Goldschmidt) give the root g and h = 1 / (2 g), a residual step rounds g,
-// another the quotient.  Zeros, negatives, subnormals, infinities and NaN take
-// the library's forms.
+// x / sqrt(a), both correctly rounded.  From one reciprocal square root: coupled
+// Newton steps (Goldschmidt) give the root g and h = 1 / (2 g), a residual step
+// rounds g.  2 h is a few units from 1 / g (g has been rounded since); a Newton
+// step rounds it, a residual step brings the quotient within a unit, and
+// another (Markstein's) rounds it.  Zeros, negatives, subnormals, infinities
+// and NaN take the library's forms.
 __device__ inline double div_sqrt(double x, double a)
 {
     if (!(a > 1e-280 && a < 1e280))
@@ -62,7 +65,10 @@ __device__ inline double div_sqrt(double x, double a)
         h = fma(h, e, h);
     }
     g = fma(fma(-g, g, a), h, g);
-    return div_by(x, g, h + h);
+    const double r = h + h, rg = fma(fma(-g, r, 1.0), r, r);
+    const double p = x * rg;
+    const double q = fma(fma(-p, g, x), rg, p);
+    return __builtin_amdgcn_class(p, kFiniteNonzero) ? fma(fma(-q, g, x), rg, q) : p;
 }
 
 }  // namespace sttrack

@@ -41,3 +41,60 @@ def test_division_of_special_values_by_a_root(lib, a):
     with np.errstate(all="ignore"):
         want = SPECIAL / np.sqrt(a)
     assert _same(_div(lib, DIV_SQRT, SPECIAL, np.full_like(SPECIAL, a)), want)
+
+
+def _hard_quotients(rng, n):
+    """(x, g), g of 53 bits, with x / g beside the midpoint of two doubles by
+    1 / (2 g) of their distance or 3 times that: x 2^54 = g m - c for an odd m
+    of 54 bits, the midpoint in units of 2^-54, and c = +-1, +-3."""
+    xs, gs = [], []
+    while len(xs) < n:
+        g, c = int(rng.integers(2**52, 2**53)) | 1, int(rng.choice([-3, -1, 1, 3]))
+        m = c * pow(g, -1, 2**54) % 2**54
+        if m >= 2**53:
+            xs.append((g * m - c) >> 54)
+            gs.append(g)
+    return np.array(xs, np.float64), np.array(gs, np.float64)
+
+
+def _hard_roots(rng, n):
+    """Doubles a whose root lies beside the midpoint of two doubles by c / (2 m):
+    a 2^55 = m^2 - c for an odd m of 54 bits and small c = 1 (mod 8), m from the
+    roots of c modulo powers of two."""
+    out = []
+    while len(out) < n:
+        c, m = 8 * int(rng.integers(-8, 9)) + 1, 2 * int(rng.integers(0, 4)) + 1
+        for k in range(3, 56):  # m^2 = c (mod 2^k) -> (mod 2^(k + 1))
+            if (m * m - c) >> k & 1:
+                m += 1 << (k - 1)
+        m = m % 2**55 if rng.integers(2) else -m % 2**55
+        if 2**53 <= m < 2**54:
+            assert (m * m - c) % 2**55 == 0
+            out.append((m * m - c) >> 55)
+    return np.array(out, np.float64) * 2.0**55
+
+
+def test_quotient_by_a_root_is_rounded(lib):
+    """The hardest quotients: the root of g^2 is g, its reciprocal has to be the
+    rounded one for the last residual to fall on the right side.  The hardest
+    roots, of 200 x each."""
+    rng = np.random.default_rng(1)
+    a = np.repeat(_hard_roots(rng, 2000), 200)
+    x = rng.standard_normal(a.size)
+    assert np.count_nonzero(_div(lib, DIV_SQRT, x, a) != x / np.sqrt(a)) == 0
+    x, g = _hard_quotients(rng, 20000)
+    a = g * g
+    assert (np.sqrt(a) == g).all()
+    assert np.count_nonzero(_div(lib, DIV_SQRT, x, a) != x / g) == 0
+    x, a = rng.standard_normal(1 << 20), np.exp(rng.uniform(-600, 600, 1 << 20))
+    assert np.count_nonzero(_div(lib, DIV_SQRT, x, a) != x / np.sqrt(a)) == 0
+
+
+def test_division_is_rounded(lib):
+    """Whole divisors up to the lags of a window (2048^2), and every mantissa."""
+    rng = np.random.default_rng(2)
+    x, n = rng.standard_normal(1 << 20) * 1e6, np.floor(np.exp(rng.uniform(0, np.log(2**22), 1 << 20)))
+    assert np.count_nonzero(_div(lib, DIV_BY, x, n) != x / n) == 0
+    n = np.arange(1.0, 2**16)
+    x = np.nextafter(n * rng.integers(1, 2**30, n.size), rng.choice([-np.inf, np.inf], n.size))
+    assert np.count_nonzero(_div(lib, DIV_BY, x, n) != x / n) == 0
