@@ -407,30 +407,6 @@ __device__ inline void refine_fine(unsigned char *scr, int t, Sync sync, double 
 // nor on one), the exponent's FP64 quotient takes the rounded product and its
 // exact residual; both are the correctly rounded ones.
 
-// exp(-t), t >= 0 or NaN, to 2^-50 (the caller rounds it to float): t log2(e)
-// split into a whole number and a rest, Taylor's series of the rest (|r| <=
-// ln 2 / 2, terms to r^12, even and odd ones in two chains).
-__device__ inline double lm_exp_neg(double t)
-{
-    t = t > 800.0 ? 800.0 : t;  // far below every float
-    const double n = __builtin_rint(t * -1.4426950408889634);
-    // ln 2 in 32 bits and the rest
-    const double r = fma(-n, -4.2009150726810846e-11, fma(-n, 0.6931471806019545, -t)), q = r * r;
-    double e = 1.0 / 479001600, o = 1.0 / 39916800;
-    e = fma(e, q, 1.0 / 3628800);
-    o = fma(o, q, 1.0 / 362880);
-    e = fma(e, q, 1.0 / 40320);
-    o = fma(o, q, 1.0 / 5040);
-    e = fma(e, q, 1.0 / 720);
-    o = fma(o, q, 1.0 / 120);
-    e = fma(e, q, 1.0 / 24);
-    o = fma(o, q, 1.0 / 6);
-    e = fma(e, q, 0.5);
-    o = fma(o, q, 1.0);
-    e = fma(e, q, 1.0);
-    return __builtin_amdgcn_ldexp(fma(o, r, e), (int)n);
-}
-
 __device__ inline void lm_coef(const float *x, const float *y, const float a[3], float alpha[3][3], float beta[3],
                                float *chisq)
 {
@@ -452,7 +428,7 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
         double arg = num * r2;
         const double whole = fma(fma(-arg, d2, num), r2, arg);
         arg = finite ? whole : arg;
-        const float ex = (float)lm_exp_neg((double)(float)arg);
+        const float ex = (float)exp(-(double)(float)arg);
         const float ymod = a[0] * ex;
         const float dyda[3] = {ex, (float)((double)(ymod * t) * r2), (float)((double)(ymod * t * t) * r3)};
         float dy = y[i] - ymod;

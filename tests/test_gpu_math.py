@@ -1,5 +1,6 @@
 """The short divisions and square roots of st_math.h on the GPU against the
-correctly rounded ones (numpy's on the host)."""
+correctly rounded ones (numpy's on the host), and the Gaussian fit's sums
+against their plain form."""
 import ctypes
 import os
 
@@ -98,3 +99,21 @@ def test_division_is_rounded(lib):
     n = np.arange(1.0, 2**16)
     x = np.nextafter(n * rng.integers(1, 2**30, n.size), rng.choice([-np.inf, np.inf], n.size))
     assert np.count_nonzero(_div(lib, DIV_BY, x, n) != x / n) == 0
+
+
+def _lm_coef(lib, y, a):
+    y, a = (np.ascontiguousarray(v, np.float32) for v in (y, a))
+    out = np.empty((2, len(a), 13), np.float32)
+    assert lib.mc_lm_coef(*(v.ctypes.data_as(ctypes.c_void_p) for v in (y, a, out)), len(a)) == 0
+    return out
+
+
+def test_fit_sums_equal_their_plain_form(lib):
+    """Amplitude, centre and width over and far beyond what a fit meets; the
+    reciprocals give the very quotients."""
+    rng = np.random.default_rng(3)
+    n = 1 << 18
+    a = np.stack([rng.uniform(-2, 3, n), rng.uniform(-8, 26, n), np.exp(rng.uniform(-3, 4, n)) * rng.choice([-1, 1], n)], 1)
+    a[n // 2:] *= 10.0 ** rng.uniform(-6, 6, (n - n // 2, 3))
+    short, plain = _lm_coef(lib, rng.uniform(0, 1, (n, 18)), a)
+    assert np.array_equal(short, plain, equal_nan=True)
