@@ -4,6 +4,7 @@
 #pragma once
 
 #include "st_common.h"
+#include "st_math.h"
 
 namespace sttrack {
 
@@ -404,9 +405,8 @@ __device__ inline void refine_fine(unsigned char *scr, int t, Sync sync, double 
 // sample's, so two FP64 reciprocals per pass replace three divisions per
 // sample: a quotient of two floats is the float rounding of the product with
 // the divisor's reciprocal (it is never within 2^-49 of a rounding boundary,
-// nor on one), the exponent's FP64 quotient takes the rounded product and its
-// exact residual; both are the correctly rounded ones.
-
+// nor on one), the exponent's FP64 quotient is div_by's; both are the correctly
+// rounded ones.
 __device__ inline void lm_coef(const float *x, const float *y, const float a[3], float alpha[3][3], float beta[3],
                                float *chisq)
 {
@@ -420,15 +420,11 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
     const float sig2i = (float)(1.0 / (double)(sg * sg));
     const float s2 = a[2] * a[2], s3 = s2 * a[2];
     const double d2 = (double)s2, r2 = 1.0 / d2, r3 = 1.0 / (double)s3;
-    const bool finite = s2 > 0.0f && s2 <= 3.402823466e38f;  // else the product is the quotient, or NaN as it is
     for (int i = 0; i < NGAUSS; i++) {
         // myGauss1D
         const float t = x[i] - a[1];
         const double num = 0.5 * (double)t * (double)t;
-        double arg = num * r2;
-        const double whole = fma(fma(-arg, d2, num), r2, arg);
-        arg = finite ? whole : arg;
-        const float ex = (float)exp(-(double)(float)arg);
+        const float ex = (float)exp(-(double)(float)div_by(num, d2, r2));
         const float ymod = a[0] * ex;
         const float dyda[3] = {ex, (float)((double)(ymod * t) * r2), (float)((double)(ymod * t * t) * r3)};
         float dy = y[i] - ymod;

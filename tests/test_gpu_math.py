@@ -117,3 +117,13 @@ def test_fit_sums_equal_their_plain_form(lib):
     a[n // 2:] *= 10.0 ** rng.uniform(-6, 6, (n - n // 2, 3))
     short, plain = _lm_coef(lib, rng.uniform(0, 1, (n, 18)), a)
     assert np.array_equal(short, plain, equal_nan=True)
+
+
+def test_fit_sums_of_special_parameters(lib):
+    """Widths and centres that are zero, infinite, NaN, or whose squares and
+    cubes leave the floats' range: what the plain quotients give."""
+    v = np.array([0.0, 1.0, -3.0, 8.5, 1e-22, 1e-15, 1e-13, 1e13, 1e19, 3e19, 3.4e38, np.inf, -np.inf, np.nan])
+    a = np.stack(np.meshgrid([1.0, 0.0, 1e30, np.inf], v, v, indexing="ij"), -1).reshape(-1, 3)
+    short, plain = _lm_coef(lib, np.random.default_rng(4).uniform(0, 1, (len(a), 18)), a)
+    bad = ~((short == plain) | (np.isnan(short) & np.isnan(plain))).all(1)
+    assert not bad.any(), a[bad]
