@@ -27,7 +27,6 @@ constexpr int kAlCols = 16;                   // columns of one pass (128 bytes 
 constexpr int kAlRows = 8;                    // rows of W per 256-thread workgroup
 constexpr int kAlBlocks = kAlW / kAlRows;     // row workgroups per try (partials of the sums)
 constexpr int kAlMagBlocks = kAlBlocks / 2;   // of k_ampl_mag (two rows per transform)
-constexpr size_t kAlLdsRows = (size_t)kAlRows * kAlPitch * sizeof(float2);
 
 // Corners, bounds and Doppler shift of the tries: state 0 (out of bounds) or
 // 2, az in units of ws.  DOP: the try's own estimate, left for the doubled

@@ -152,10 +152,6 @@ __device__ inline void inv_pair(float2 (&x)[W / 2], int h)
 // lane h holds inputs qblk(h) * 32 + n, the same two exchanges in the
 // opposite order (decimation in frequency), then the 32-point transforms;
 // lane h leaves with outputs 4j + h.
-// exp(+2 pi i j / 256), j = 0..31 (the polyphase factors at w = 128)
-constexpr float kTw256Re[32] = {0x1p+0f, 0x1.ffd886p-1f, 0x1.ff621ep-1f, 0x1.fe9cdap-1f, 0x1.fd88dap-1f, 0x1.fc2648p-1f, 0x1.fa7558p-1f, 0x1.f8765p-1f, 0x1.f6297cp-1f, 0x1.f38f3ap-1f, 0x1.f0a7fp-1f, 0x1.ed740ep-1f, 0x1.e9f416p-1f, 0x1.e6288ep-1f, 0x1.e2121p-1f, 0x1.ddb13cp-1f, 0x1.d906bcp-1f, 0x1.d4134ep-1f, 0x1.ced7bp-1f, 0x1.c954b2p-1f, 0x1.c38b3p-1f, 0x1.bd7c0ap-1f, 0x1.b72834p-1f, 0x1.b090a6p-1f, 0x1.a9b662p-1f, 0x1.a29a7ap-1f, 0x1.9b3e04p-1f, 0x1.93a224p-1f, 0x1.8bc806p-1f, 0x1.83b0ep-1f, 0x1.7b5df2p-1f, 0x1.72d084p-1f};
-constexpr float kTw256Im[32] = {0x0p+0f, 0x1.92156p-6f, 0x1.91f66p-5f, 0x1.2d520ap-4f, 0x1.917a6cp-4f, 0x1.f564e6p-4f, 0x1.2c8106p-3f, 0x1.5e2144p-3f, 0x1.8f8b84p-3f, 0x1.c0b826p-3f, 0x1.f19f98p-3f, 0x1.111d26p-2f, 0x1.294062p-2f, 0x1.4135cap-2f, 0x1.58f9a8p-2f, 0x1.708854p-2f, 0x1.87de2ap-2f, 0x1.9ef794p-2f, 0x1.b5d1p-2f, 0x1.cc66eap-2f, 0x1.e2b5d4p-2f, 0x1.f8ba4ep-2f, 0x1.07387ap-1f, 0x1.11eb36p-1f, 0x1.1c73b4p-1f, 0x1.26d054p-1f, 0x1.30ff8p-1f, 0x1.3affa2p-1f, 0x1.44cf32p-1f, 0x1.4e6cacp-1f, 0x1.57d694p-1f, 0x1.610b76p-1f};
-
 __device__ inline int qblk(int h) { return ((h & 1) << 1) | (h >> 1); }
 
 // Value of lane ^ 2 via DPP quad_perm [2,3,0,1].
