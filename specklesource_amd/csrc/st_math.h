@@ -7,10 +7,10 @@
 namespace sttrack {
 
 // sqrtf for finite x >= 2^-96: the rounded product of x and its hardware
-// reciprocal square root, corrected by half its exact residual times the
-// latter.  Equal to sqrtf(x) at every such float (all 1.88e9 compared on
-// gfx950); five instructions against nine for the hardware root with its two
-// one-ulp tests, sixteen for sqrtf.
+// reciprocal square root, then one Newton step by its exact residual (Markstein's
+// correction of a root).  Correctly rounded at every such float (the test
+// compares all 1.88e9); five instructions against nine for the hardware root
+// with its two one-ulp tests, sixteen for sqrtf.
 __device__ inline float sqrt_rn_normal(float x)
 {
     const float y = __builtin_amdgcn_rsqf(x);

@@ -88,14 +88,65 @@ def test_constant_windows(device, monkeypatch, wa, ulps):
         assert np.array_equal(f.diag[k][1], s.diag[k][1]), k
 
 
-def test_one_try_and_no_try(device):
+def _both_paths(device, monkeypatch, pid, p):
+    f = device.speckle_track(pid, p, diag=True)
+    monkeypatch.setenv("SPECKLE_AMD_PATH", "staged")
+    s = device.speckle_track(pid, p, diag=True)
+    monkeypatch.delenv("SPECKLE_AMD_PATH")
+    assert (f.nAmp, f.nAmpL, f.nFail) == (s.nAmp, s.nAmpL, s.nFail)
+    for k in ("offR", "offA", "azd", "type"):
+        assert np.array_equal(getattr(f, k), getattr(s, k)), k
+    for k in ("peakI", "peakJ", "fineI", "fineJ", "sigRg", "sigAz", "peakGap", "fineGap"):
+        for t in (1, 2):
+            assert np.array_equal(f.diag[k][t], s.diag[k][t]), (k, t)
+    assert np.allclose(f.corr, s.corr, rtol=2**-23, atol=0)  # as in test_fused_tries_equal_staged_tries
+    return f
+
+
+@pytest.mark.parametrize("wa,n,step", [(16, 120, 4), (32, 64, 7), (64, 32, 20)])
+def test_several_tries_per_workgroup(device, monkeypatch, wa, n, step):
+    """More tries than resident workgroups (at most 4096, 1024 and 256 of them),
+    so that each takes three or four one after the other, with tries that leave
+    early among them: windows outside the image, windows without data."""
+    a, b = _pair(n * step - 9, n * step - 21, wa, abi.ST_SAMPLE_C64)
+    for x in (a, b):
+        x[60:150, 70:200] = 0
+    p = small_params(wa, n * step, n * step, step=step, wRa=wa, wAa=wa, noComplex=1, rStart=0, aStart=0, nR=n, nA=n,
+                     rShiftPoly=[1.0, 0, 0], aShiftPoly=[-1.0, 0, 0])
+    pid = device.upload_pair(a, b)
+    try:
+        f = _both_paths(device, monkeypatch, pid, p)
+    finally:
+        device.release_pair(pid)
+    matched = (f.diag["peakI"][1] != -2000).mean()  # tries that reached the correlation
+    assert n * n > 2.5 * {16: 4096, 32: 1024, 64: 256}[wa]
+    assert 0.4 < matched < 0.95 and f.nAmp > 100, matched
+
+
+@pytest.mark.parametrize("w,wa", [(64, 64), (64, 128)])
+def test_gauss_fits_on_the_128_sample_passes(device, monkeypatch, w, wa):
+    """-gauss: the fit reads the surface that the 128 sample passes leave, of the
+    doubled window or of the small one."""
+    n = 14 if wa < 128 else 9
+    a, b = _pair(n * wa + 37, n * wa + 11, 3 + wa, abi.ST_SAMPLE_C64)
+    p = small_params(w, n * wa, n * wa, step=wa - 3, wRa=wa, wAa=wa, noComplex=1, gaussFlag=1, rStart=wa, aStart=wa,
+                     nR=n - 1, nA=n - 1, rShiftPoly=[1.0, 0, 0], aShiftPoly=[-1.0, 0, 0])
+    pid = device.upload_pair(a, b)
+    try:
+        f = _both_paths(device, monkeypatch, pid, p)
+    finally:
+        device.release_pair(pid)
+    assert f.nAmp > 0 and (f.nAmpL > 0 or wa == 128)
+
+
+def test_one_try_and_no_try(device, monkeypatch):
     """A single point, and a grid whose windows all leave the image."""
     a, b = _pair(160, 160, 3, abi.ST_SAMPLE_C64)
     pid = device.upload_pair(a, b)
     try:
         p = small_params(32, 160, 160, noComplex=1, nR=1, nA=1, rStart=50, aStart=40)
-        g = device.speckle_track(pid, p)
-        assert g.type.shape == (1, 1)
+        g = _both_paths(device, monkeypatch, pid, p)
+        assert g.type.shape == (1, 1) and g.diag["peakI"][1][0, 0] != -2000
         p = small_params(32, 160, 160, noComplex=1, nR=3, nA=2, rShiftPoly=[4000.0, 0, 0])
         g = device.speckle_track(pid, p)
         assert (g.type == 0).all() and g.nAmp == g.nAmpL == 0

@@ -51,6 +51,19 @@ def test_ls_schedules(device, oracle32, monkeypatch, iters):
     assert np.array_equal(ga["X"], oa["X"]) and np.array_equal(ga["Y"], oa["Y"])
 
 
+@pytest.mark.parametrize("iters", ["48", "0"])
+def test_ls_largest_box(device, oracle32, monkeypatch, iters):
+    """A 45 x 45 box: the fixpoint kernel's tile with the type plane takes 67 KB
+    of LDS; and the wavefront kernel."""
+    monkeypatch.setenv("SPECKLE_AMD_CULL_ITERS", iters)
+    X, Y, typ = _ls_grid(49, 70, seed=9, outlier_frac=0.15)
+    (gc, ga), (oc, oa) = _pair(X, Y, typ, bR=45, bA=45, nGood=60)
+    device.cull("st_cull_ls_data", gc)
+    oracle32.cull("st_cull_ls_data", oc)
+    assert gc.nCulled == oc.nCulled > 0
+    assert np.array_equal(ga["X"], oa["X"]) and np.array_equal(ga["Y"], oa["Y"])
+
+
 def test_ls_nodata_value(device, oracle32):
     X, Y, typ = _ls_grid(40, 40, seed=6)
     Y[10:14, 10:30] = -1000.0

@@ -1,6 +1,6 @@
 """The short divisions and square roots of st_math.h on the GPU against the
 correctly rounded ones (numpy's on the host), and the Gaussian fit's sums
-against their plain form."""
+and 3 x 3 solve against their plain forms."""
 import ctypes
 import os
 
@@ -127,3 +127,41 @@ def test_fit_sums_of_special_parameters(lib):
     short, plain = _lm_coef(lib, np.random.default_rng(4).uniform(0, 1, (len(a), 18)), a)
     bad = ~((short == plain) | (np.isnan(short) & np.isnan(plain))).all(1)
     assert not bad.any(), a[bad]
+
+
+def test_every_square_root_of_the_short_form(lib):
+    """All floats from 2^-96 to the largest, against the rounded FP64 root."""
+    bad = ctypes.c_ulonglong(1)
+    assert lib.mc_sqrt(0x0F800000, 0x7F800000, ctypes.byref(bad)) == 0
+    assert bad.value == 0
+
+
+def test_range_test_of_the_short_square_root(lib):
+    """One value of a wave outside [2^-96, FLT_MAX], in either register and any
+    lane, sends the whole wave to the full form; values at the ends do not."""
+    inside = np.array([2.0**-96, 1.0, np.finfo(np.float32).max], np.float32)
+    outside = np.array([0.0, 1e-45, np.nextafter(np.float32(2.0**-96), np.float32(0)), np.inf, np.nan], np.float32)
+    x = np.random.default_rng(5).choice(inside, (2 * 64 * len(outside) + 2, 64, 2))
+    for k, v in enumerate(outside):
+        for lane in range(64):
+            for reg in range(2):
+                x[(k * 64 + lane) * 2 + reg, lane, reg] = v
+    r = np.empty(x.shape[:2], np.int32)
+    assert lib.mc_needs_full(*(v.ctypes.data_as(ctypes.c_void_p) for v in (x, r)), len(x)) == 0
+    assert (r[:-2] != 0).all() and (r[-2:] == 0).all()
+
+
+def test_solve3_equals_its_plain_form(lib):
+    """Random systems, symmetric ones as the fit's, ties of the pivots, singular
+    ones, infinities and NaN."""
+    rng = np.random.default_rng(6)
+    n = 1 << 16
+    a = rng.standard_normal((4, n, 12)) * 10.0 ** rng.uniform(-4, 4, (4, n, 12))
+    a[1, :, 3], a[1, :, 6], a[1, :, 7] = a[1, :, 1], a[1, :, 2], a[1, :, 5]
+    a[2] = rng.integers(-2, 3, (n, 12))
+    a[3] = rng.choice([0.0, 1.0, -1.0, 1e30, 1e-40, np.inf, np.nan], (n, 12), p=[.2, .3, .2, .1, .1, .05, .05])
+    a = np.ascontiguousarray(a.reshape(-1, 12), np.float32)
+    out = np.empty((2, len(a), 4), np.float32)
+    assert lib.mc_solve3(*(v.ctypes.data_as(ctypes.c_void_p) for v in (a, out)), len(a)) == 0
+    assert np.array_equal(out[0], out[1], equal_nan=True)
+    assert 0.2 < out[0, 2 * n:3 * n, 0].mean() < 0.95
