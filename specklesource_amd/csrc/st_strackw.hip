@@ -661,12 +661,9 @@ __global__ void __launch_bounds__(256) k_w_ncc(WPar p, WBatch Bt, WfBatch F, int
                                        (c < 0 ? c + p.W_R : c)];
                 v = b & 1 ? xv.y : xv.x;
             }
-            const double m = div_by(P1[p.wR2] - P1[0], N, rN);
-            const double sig = div_by(P2[p.wR2] - P2[0], N - 1., rN1) - m * m;
             const float mag = sqrtf(v * v);  // = (float)sqrt((double)(v * v)), bit for bit
-            double cr = (double)mag * p.scaleW;
-            cr = cr - meanR * m;
-            cr = div_sqrt(cr, sigmaR * sig);
+            const double cr = ncc_value((double)mag * p.scaleW, meanR, sigmaR, P1[p.wR2] - P1[0], P2[p.wR2] - P2[0], N,
+                                        rN, rN1);
             Bt.cr[e0 + e] = (float)cr;
             if (l >= -sA && l <= sA && c >= -sR && c <= sR) {
                 if (cr > best) {

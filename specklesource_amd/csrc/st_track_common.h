@@ -405,8 +405,8 @@ __device__ inline void refine_fine(unsigned char *scr, int t, Sync sync, double 
 // sample's, so two FP64 reciprocals per pass replace three divisions per
 // sample: a quotient of two floats is the float rounding of the product with
 // the divisor's reciprocal (it is never within 2^-49 of a rounding boundary,
-// nor on one), the exponent's FP64 quotient is div_by's; both are the correctly
-// rounded ones.
+// nor on one), the exponent's FP64 quotient takes the rounded product and its
+// exact residual; both are the correctly rounded ones.
 __device__ inline void lm_coef(const float *x, const float *y, const float a[3], float alpha[3][3], float beta[3],
                                float *chisq)
 {
@@ -424,7 +424,10 @@ __device__ inline void lm_coef(const float *x, const float *y, const float a[3],
         // myGauss1D
         const float t = x[i] - a[1];
         const double num = 0.5 * (double)t * (double)t;
-        const float ex = (float)exp(-(double)(float)div_by(num, d2, r2));
+        double arg = num * r2;
+        if (finite_nonzero(arg))  // else it is the quotient, and has no residual
+            arg = fma(fma(-arg, d2, num), r2, arg);
+        const float ex = (float)exp(-(double)(float)arg);
         const float ymod = a[0] * ex;
         const float dyda[3] = {ex, (float)((double)(ymod * t) * r2), (float)((double)(ymod * t * t) * r3)};
         float dy = y[i] - ymod;

@@ -192,6 +192,29 @@ extern "C" int mc_div(int kind, const double *x, const double *n, double *q, int
     return e == hipSuccess ? hipMemcpy(q, dq.p, count * sizeof(double), hipMemcpyDeviceToHost) : e;
 }
 
+// in [count][6]: c, mean, var, s1, s2, n
+__global__ void k_ncc(const double *in, double *out, int count)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) {
+        const double *v = in + 6 * (size_t)i;
+        out[i] = ncc_value(v[0], v[1], v[2], v[3], v[4], v[5], 1.0 / v[5], 1.0 / (v[5] - 1.0));
+    }
+}
+
+extern "C" int mc_ncc(const double *in, double *out, int count)
+{
+    Buf<double> di(6 * (size_t)count), dout(count);
+    if (!di.p || !dout.p)
+        return hipErrorOutOfMemory;
+    hipError_t e = hipMemcpy(di.p, in, 6 * sizeof(double) * count, hipMemcpyHostToDevice);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_ncc, dim3((count + 255) / 256), dim3(256), 0, 0, di.p, dout.p, count);
+        e = hipGetLastError();
+    }
+    return e == hipSuccess ? hipMemcpy(out, dout.p, sizeof(double) * count, hipMemcpyDeviceToHost) : e;
+}
+
 extern "C" int mc_lm_coef(const float *y, const float *a, float *out, int count)
 {
     Buf<float> dy((size_t)NGAUSS * count), da(3 * (size_t)count), dout(26 * (size_t)count);

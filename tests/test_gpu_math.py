@@ -24,24 +24,38 @@ def _div(lib, kind, x, n):
     return q
 
 
-def _same(a, b):
-    """Equal, signs of zeros and places of NaN included."""
-    return np.array_equal(a, b, equal_nan=True) and np.array_equal(np.signbit(a), np.signbit(b))
+def _ncc(lib, v):
+    v = np.ascontiguousarray(v, np.float64)
+    out = np.empty(len(v))
+    assert lib.mc_ncc(*(x.ctypes.data_as(ctypes.c_void_p) for x in (v, out)), len(v)) == 0
+    return out
 
 
-SPECIAL = np.array([0.0, -0.0, np.inf, -np.inf, 1.0, -1.0, 3e38, 1e-45])
+def _ncc_plain(v):
+    c, mean, var, s1, s2, n = v.T
+    m = s1 / n
+    return (c - mean * m) / np.sqrt(var * (s2 / (n - 1) - m * m))
 
 
-@pytest.mark.parametrize("n", [1.0, 3.0, 65536.0, 147455.0])
-def test_division_of_special_values(lib, n):
-    assert _same(_div(lib, DIV_BY, SPECIAL, np.full_like(SPECIAL, n)), SPECIAL / n)
-
-
-@pytest.mark.parametrize("a", [4.0, 1e-280, 1e280, 1e-300, 0.0, np.inf, 2.0])
-def test_division_of_special_values_by_a_root(lib, a):
+def test_correlation_of_special_values(lib):
+    """Sums, means and variances that are zero, infinite, NaN or near the ends of
+    the range: the plain quotients' values, infinities among them."""
+    x = [0.0, 3.0, -2.5, 1e-140, 1e150, 1e300, np.inf, -np.inf, np.nan]
+    v = np.stack(np.meshgrid(x, x, x, x, x, [65536.0, 97 * 31.0], indexing="ij"), -1).reshape(-1, 6)
     with np.errstate(all="ignore"):
-        want = SPECIAL / np.sqrt(a)
-    assert _same(_div(lib, DIV_SQRT, SPECIAL, np.full_like(SPECIAL, a)), want)
+        want = _ncc_plain(v)
+    got = _ncc(lib, v)
+    assert np.array_equal(got, want, equal_nan=True), v[~((got == want) | (np.isnan(got) & np.isnan(want)))][:5]
+    assert np.isinf(want).any() and np.isnan(want).any()
+
+
+def test_correlation_is_the_plain_one(lib):
+    rng = np.random.default_rng(7)
+    n = np.floor(rng.uniform(3, 200, 1 << 20)) * np.floor(rng.uniform(3, 200, 1 << 20))
+    mean = rng.uniform(0, 3, n.size) * 10.0 ** rng.uniform(-6, 6, n.size)
+    v = np.stack([mean * mean * rng.uniform(0, 2, n.size), mean, mean**2 * rng.uniform(0.01, 1, n.size), n * mean,
+                  n * mean**2 * rng.uniform(1.01, 2, n.size), n], 1)
+    assert np.count_nonzero(_ncc(lib, v) != _ncc_plain(v)) == 0
 
 
 def _hard_quotients(rng, n):
