@@ -26,9 +26,9 @@
 //   F  range inverse, two rows per transform, |s|, coarse top two
 // The refinement and the width samples follow in k_cpx_refine.
 //
-// Bound: FP32 VALU issue (the VALU is busy 85 % of the time at ws = 32, 77 %
-// at 64).  Per try, 28 665 tries at ws = 32: 35 ns (the staged kernels 146
-// ns); 9 744 at ws = 64: 160 ns (600 ns).
+// Bound: FP32 VALU issue (a VALU instruction on 83 % of the SIMDs' cycles at
+// ws = 32, on 76 % at 64).  Per try, 28 665 tries at ws = 32: 34 ns (the staged
+// kernels 143 ns); 9 744 at ws = 64: 164 ns (600 ns).
 
 // Workgroup geometry for W = 2 ws: U = 2 units of eight values per lane, so
 // that the half-size passes (A, B, F) occupy every lane with one.  Measured at

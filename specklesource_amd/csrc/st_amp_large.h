@@ -19,9 +19,10 @@
 // .. k_amp_rowmag): bit-identical surfaces.  Every pass reads and writes whole
 // 128-byte segments; columns go through LDS 16 at a time.
 //
-// Bound: HBM traffic (5.2 MB per try at 4.4 TB/s) and FP32 VALU issue, about
-// equally.  6 732 doubled windows: 2.5 us per try with the staged kernels,
-// 1.2 us with these.
+// Bound: HBM traffic: 4.7 MB per try (writes as counted, reads as laid out) at
+// 4.0 TB/s; k_ampl_det also issues a VALU instruction on 77 % of the SIMDs'
+// cycles, the others on 30 to 49 %.  6 732 doubled windows: 2.4 us per try with
+// the staged kernels, 1.2 us with these.
 constexpr int kAlWS = 128, kAlW = 256, kAlPitch = kAlW + kAlW / 8 + 1;
 constexpr int kAlCols = 16;                   // columns of one pass (128 bytes of a row)
 constexpr int kAlRows = 8;                    // rows of W per 256-thread workgroup

@@ -529,7 +529,7 @@ __device__ inline void wave_scan(double (&x)[n])
 // Bound: FP64 issue and the latency between the two barriers of a round.  The
 // next rows' samples are loaded before the lags are computed, divisions by
 // constants and by the root take three and some twenty operations.  576 patches
-// of 513^2 lags (768 columns): 1.30 ms; 2.43 with two LDS passes per prefix,
+// of 513^2 lags (768 columns): 1.37 ms; 2.43 with two LDS passes per prefix,
 // shuffles through LDS for the scans and for every row's two best, and four
 // barriers per round.
 template <int PER, int STEP, bool FIXED>
