@@ -3,6 +3,7 @@ correctly rounded ones (numpy's on the host), and the Gaussian fit's sums
 and 3 x 3 solve against their plain forms."""
 import ctypes
 import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -14,7 +15,11 @@ DIV_BY, DIV_SQRT = 0, 1
 
 @pytest.fixture(scope="module")
 def lib(device):
-    return ctypes.CDLL(os.path.join(os.path.dirname(__file__), "native", "_build", "libmath_check.so"))
+    native = os.path.join(os.path.dirname(os.path.abspath(__file__)), "native")
+    so = os.path.join(native, "_build", "libmath_check.so")
+    if not os.path.exists(so):  # build() makes it
+        subprocess.run(["make", "-s", "-C", native], check=True)
+    return ctypes.CDLL(so)
 
 
 def _div(lib, kind, x, n):
